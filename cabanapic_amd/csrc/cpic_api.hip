@@ -12,10 +12,12 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/cabanapic_amd.h"
 #include "cpic_push_kernels.h"
+#include "cpic_split_kernels.h"
 #include "cpic_tangent_kernels.h"
 #include "cpic_adjoint_kernels.h"
 
@@ -99,6 +101,13 @@ struct ColumnSet {
   // it writes a record addressed to a cell of the group, cleared by the
   // second, whose waves without a mark have nothing to do
   int* rec_flags = nullptr;
+  // per group, in the same allocation: rows its columns used in the last push
+  // and particles that took the move_p branch
+  int* grp_rows = nullptr;
+  int* grp_movers = nullptr;
+  // rows that pass 2 took, [MW][nc_pad], for columns of more than
+  // kTakenWords words only
+  unsigned long long* taken = nullptr;
 };
 
 constexpr int kStatusStride = 64;  // ints per status line (256 bytes)
@@ -111,9 +120,9 @@ struct cpic_context : ColumnSet {
   long nc_pad = 0;  // interior cells rounded up to whole blocks (kBlock lanes)
   long cap = 0;     // particle capacity declared at creation
   long column_rows = 0;  // requested rows per column (0 = automatic)
-  int* occ_host = nullptr;        // pinned copies of the last push's error flags and max_count
-  hipEvent_t occ_event = nullptr;  // recorded after those copies
-  bool occ_pending = false;        // a copy is in flight
+  PushStatus* push_host = nullptr;  // pinned: status of the last push, written by the device
+  int push_seq = 0;                 // number of the last push launched
+  bool push_pending = false;        // its status has not been looked at
   long np = 0;      // particles resident (conserved by the push)
   Grid grid{};
   CellGrid cg{};
@@ -123,22 +132,19 @@ struct cpic_context : ColumnSet {
   long pushes = 0;         // pushes since the last upload (the first of every
                            // compaction interval packs the columns)
   // device status words, one allocation (status), each on its own 256-byte
-  // line (every wave reads the error flags while pass 1's waves update the
-  // counters atomically; sharing a line slowed the step by 20 us):
-  // [0] error flags (err), [kStatusStride] largest column occupancy seen by
-  // the last push (max_count), [2 kStatusStride] particles that left their
-  // cell (movers), [3 kStatusStride] overflow records (ovf_count).  A push
-  // clears the three counters with one launch and the host reads err and
-  // max_count back with one copy.
+  // line: [0] error flags (err), [kStatusStride] particles that left their
+  // cell in a tangent push (movers), [2 kStatusStride] overflow records
+  // (ovf_count, zero between pushes)
   int* status = nullptr;
   unsigned int* ovf_count = nullptr;
-  int* max_count = nullptr;
 
   void* fields = nullptr;
   void* interp = nullptr;
   void* acc = nullptr;             // slot-major [12][Ng]
   bool acc_ghosts_zero = true;     // ghost accumulators known to be zero
-  double* partials = nullptr;  // reduction partials
+  double* partials = nullptr;  // reduction partials: [partial_rows][n_partials][2] field
+                               // energies of steps in turn, [n_partials] kinetic
+  int partial_rows = 1;
   double* red_out = nullptr;   // [E, B, KE]
   int* err = nullptr;
   unsigned int* movers = nullptr;
@@ -299,17 +305,51 @@ ColState<R> col_state(cpic_context* c, int from) {
   return cs;
 }
 
+// Waves that share a group of 64 cells in pass 1 and in pass 2: 8 where the
+// groups alone do not fill the chip (1024 SIMDs), else 4 and 2.  Pass 1 / pass
+// 2 in us, with 2, 4 and 8 waves: 32^3 cells x 32 (512 groups) 45 29 25 / 23
+// 18 16; 48^3 x 32 (1728) 87 85 85 / 44 46 58; 128^3 x 32 (32768) 1324 1281
+// 1347 / 724 726 998; 1D, 32 cells x 64 in FP64, 95 58 42 / 41 31 26.  (One
+// wave: 1359 / 731 at 128^3.)
+struct SplitWaves {
+  int push, arrive;
+};
+SplitWaves split_waves(const cpic_context* c) {
+  if (cdiv(c->nc, 64) <= 512) return {8, 8};
+  return {4, 2};
+}
+
+// Whether this push packs the columns: every interval-th one that the caller
+// names, by default every kCompactInterval-th of a grid that fills the chip.
+// Packing walks a column with one wave, and arrivals keep filling the lowest
+// holes, so that the columns of a small grid stay short without it.
+bool packs_now(cpic_context* c, int interval) {
+  const long n = c->pushes++;
+  if (interval <= 0 && cdiv(c->nc, 64) < 2048) return false;
+  return n % (interval > 0 ? interval : kCompactInterval) == 0;
+}
+
+template <class R, bool K>
+void launch_push_split(cpic_context* c, const PushPass<R>& p, int S) {
+  const int groups = cdiv(c->nc, 64);
+  S == 4 ? k_push_split<R, K, 4><<<groups, 64 * 4, 0, c->stream>>>(p)
+         : k_push_split<R, K, 8><<<groups, 64 * 8, 0, c->stream>>>(p);
+}
+template <class R, bool K>
+void launch_arrive_split(cpic_context* c, const ArrivePass<R>& a, int S) {
+  const int groups = cdiv(c->nc, 64);
+  S == 2 ? k_arrive_split<R, K, 2><<<groups, 64 * 2, 0, c->stream>>>(a)
+         : k_arrive_split<R, K, 8><<<groups, 64 * 8, 0, c->stream>>>(a);
+}
+
 // push + move_p + deposit: pass 1, three finishing passes, spill fallback.
 // accumulate = 1 adds to the accumulators as the reference's push does;
 // accumulate = 0 overwrites them (valid right after a clear).  gather: where
 // pass 1 takes the interpolators from (the array, or the fields).
 template <class R>
 int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, int accumulate,
-               int compact, int gather = kGatherRead) {
+               bool compact, int gather = kGatherRead) {
   StageTimer t(c, CPIC_STAGE_PUSH);
-  int s;
-  // max_count, movers and ovf_count (and the unused words between them)
-  if ((s = fill_zero<int>(c, c->max_count, 2 * kStatusStride + 1))) return s;
   if (c->np == 0) return t.finish();
   if (c->D == 0) return fail(CPIC_ERR_INVALID, "particles resident without columns");
   const int blocks = cdiv(c->nc, kBlock);
@@ -335,18 +375,19 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   p.qsp = qsp;
   p.accumulate = accumulate;
   p.err = c->err;
-  p.movers = c->movers;
-  p.max_count = c->max_count;
-  // k_push_rows keeps every particle in its row; k_push_pass packs the
-  // columns.  The row stores of k_push_rows address one column group with
+  p.grp_rows = c->grp_rows;
+  p.grp_movers = c->grp_movers;
+  // k_push_split keeps every particle in its row; k_push_pass packs the
+  // columns.  The row stores of k_push_split address one column group with
   // 32-bit byte offsets; columns too deep for that are packed at every push.
   const bool group_fits = (int64_t)c->D * 64 * kSlotLen * (int64_t)sizeof(R) < INT32_MAX;
+  const SplitWaves waves = split_waves(c);
   if (compact || !group_fits)
     c->compensated ? k_push_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
                    : k_push_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
   else
-    c->compensated ? k_push_rows<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
-                   : k_push_rows<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
+    c->compensated ? launch_push_split<R, true>(c, p, waves.push)
+                   : launch_push_split<R, false>(c, p, waves.push);
   CHECK_LAUNCH();
 
   // the streak after the 1st crossing, found through the departure masks
@@ -354,6 +395,7 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   ar.cs = cs;
   ar.dep = c->dep;
   ar.dep_words = c->dep_words;
+  ar.taken = c->taken;
   ar.out = L2;
   ar.ovf = ovf;
   ar.acc = (R*)c->acc;
@@ -364,8 +406,8 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   ar.cdt_dz = cdt_dz;
   ar.qsp = qsp;
   ar.err = c->err;
-  c->compensated ? k_arrive_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(ar)
-                 : k_arrive_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(ar);
+  c->compensated ? launch_arrive_split<R, true>(c, ar, waves.arrive)
+                 : launch_arrive_split<R, false>(c, ar, waves.arrive);
   CHECK_LAUNCH();
 
   // the streaks after the 2nd and 3rd crossings, from the record lists
@@ -396,13 +438,19 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   return t.finish();
 }
 
+// real_t products, double quotient, stored as real_t (accumulator.cpp:66-68)
+template <class R>
+void unload_scales(R dx, R dy, R dz, R dt, R& cx, R& cy, R& cz) {
+  cx = 0.25 / (dy * dz * dt);
+  cy = 0.25 / (dz * dx * dt);
+  cz = 0.25 / (dx * dy * dt);
+}
+
 template <class R>
 int stage_unload(cpic_context* c, R dx, R dy, R dz, R dt) {
   StageTimer t(c, CPIC_STAGE_UNLOAD);
-  // real_t products, double quotient, stored as real_t (accumulator.cpp:66-68)
-  const R cx = 0.25 / (dy * dz * dt);
-  const R cy = 0.25 / (dz * dx * dt);
-  const R cz = 0.25 / (dx * dy * dt);
+  R cx, cy, cz;
+  unload_scales<R>(dx, dy, dz, dt, cx, cy, cz);
   const long n = (c->nx + 1) * (c->ny + 1) * (c->nz + 1);
   k_unload<R><<<cdiv(n, kBlock), kBlock, 0, c->stream>>>((R*)c->fields, (const R*)c->acc, c->grid,
                                                          cx, cy, cz);
@@ -471,6 +519,14 @@ int stage_advance_e(cpic_context* c, R px, R py, R pz, R dt_eps0) {
   return t.finish();
 }
 
+// The first rows sets of field-energy partials, blocks each, summed into out,
+// out + stride, ...
+int launch_energy_rows(cpic_context* c, int rows, int blocks, double* out, int stride) {
+  k_reduce_final<2><<<rows, kBlock, 0, c->stream>>>(c->partials, blocks, 0.5, 0.5, out, stride);
+  CHECK_LAUNCH();
+  return CPIC_OK;
+}
+
 // E and B energies into out[0..1] (device), FP64.
 template <class R>
 int launch_field_energy(cpic_context* c, double* out) {
@@ -484,14 +540,12 @@ int launch_field_energy(cpic_context* c, double* out) {
     k_field_energy_partial<R><<<blocks, kBlock, 0, c->stream>>>((const R*)c->fields, c->grid,
                                                                 c->partials);
   CHECK_LAUNCH();
-  k_reduce_final<2><<<1, kBlock, 0, c->stream>>>(c->partials, blocks, 0.5, 0.5, out);
-  CHECK_LAUNCH();
-  return CPIC_OK;
+  return launch_energy_rows(c, 1, blocks, out, 0);
 }
 
 template <class R>
 int launch_kinetic(cpic_context* c, double scale, double* out) {
-  double* part = c->partials + 2 * (size_t)c->n_partials;
+  double* part = c->partials + 2 * (size_t)c->partial_rows * c->n_partials;
   int blocks = 1;
   if (c->D > 0 && c->np > 0) {
     blocks = std::max(1, std::min(cdiv(c->nc, kBlock), c->n_partials));
@@ -518,7 +572,8 @@ void free_column_set(ColumnSet& s) {
     if (s.cnt[b]) (void)hipFree(s.cnt[b]);
     if (s.mask[b]) (void)hipFree(s.mask[b]);
   }
-  void* ptrs[] = {s.rec1, s.rec2, s.rc1, s.rc2, s.ovf_rec, s.ovf_cell, s.dep, s.dep_words};
+  void* ptrs[] = {s.rec1,     s.rec2, s.rc1,       s.rc2,  s.ovf_rec,
+                  s.ovf_cell, s.dep,  s.dep_words, s.taken};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   s = ColumnSet{};
@@ -551,14 +606,19 @@ int alloc_column_set(cpic_context* c, int D, int M1, int M2, ColumnSet& out) {
     if ((t = alloc(&s.ovf_rec, (size_t)record_bytes(c->real_size) * s.ovf_cap))) return t;
     if ((t = alloc((void**)&s.ovf_cell, sizeof(int) * s.ovf_cap))) return t;
     if ((t = alloc((void**)&s.dep, sizeof(unsigned long long) * kDepMasks * words))) return t;
-    if ((t = alloc((void**)&s.dep_words, sizeof(int) * 2 * (c->nc_pad / 64)))) return t;
-    s.rec_flags = s.dep_words + c->nc_pad / 64;
+    const size_t groups = c->nc_pad / 64;
+    if ((t = alloc((void**)&s.dep_words, sizeof(int) * 4 * groups))) return t;
+    if (s.MW > kTakenWords)
+      if ((t = alloc((void**)&s.taken, sizeof(unsigned long long) * words))) return t;
+    s.rec_flags = s.dep_words + groups;
+    s.grp_rows = s.dep_words + 2 * groups;
+    s.grp_movers = s.dep_words + 3 * groups;
     for (int b = 0; b < 2; ++b) {
       if ((t = fill_zero<int>(c, s.cnt[b], c->nc_pad))) return t;
       if ((t = fill_zero<unsigned long long>(c, s.mask[b], words))) return t;
     }
     if ((t = fill_zero<unsigned long long>(c, s.dep, kDepMasks * words))) return t;
-    if ((t = fill_zero<int>(c, s.dep_words, 2 * (c->nc_pad / 64)))) return t;
+    if ((t = fill_zero<int>(c, s.dep_words, 4 * groups))) return t;
     return CPIC_OK;
   };
   if (int t = run()) {
@@ -610,28 +670,50 @@ int check_device_errors(cpic_context* c) {
 }
 
 // ---- column headroom -------------------------------------------------------
-// Each push copies its largest input column occupancy (rows in use) and the
-// device error flags to pinned host memory.  Before the next push the host
-// reads the copies (one step behind, so the GPU does not idle).  A set flag
-// fails the push: the kernels of a push also return at once when a flag is
-// set, so pushes already queued behind a failed one change nothing.  A
-// column within max(8, D/4) rows of its capacity makes the host re-lay the
-// columns out on the device with 1.5x the rows, so that particles bunching
-// in one cell (a nonlinear two-stream phase reaches 4x the mean count) do
-// not overflow it.  A push that overflows anyway fails with kErrColumnFull.
+// After each push the device writes its largest input column occupancy (rows
+// in use) and the error flags to pinned host memory (PushStatus).  Before the
+// next push the host looks at them, one step behind, so the GPU does not
+// idle.  A set flag fails the push; the kernels of a push also return at once
+// when a flag is set, so pushes already queued behind a failed one change
+// nothing.  A column within max(8, D/4) rows of its capacity makes the host
+// re-lay the columns out on the device with 1.5x the rows, so that particles
+// bunching in one cell (a nonlinear two-stream phase reaches 4x the mean
+// count) do not overflow it.  A push that overflows anyway fails with
+// kErrColumnFull.
 
-int note_occupancy(cpic_context* c) {
-  if (c->D == 0 || c->np == 0) return CPIC_OK;
-  if (!c->occ_host) {
-    HIP_TRY(hipHostMalloc((void**)&c->occ_host, (kStatusStride + 1) * sizeof(int),
-                          hipHostMallocDefault));
-    HIP_TRY(hipEventCreateWithFlags(&c->occ_event, hipEventDisableTiming));
+int column_groups(const cpic_context* c) { return (int)(c->nc_pad / 64); }
+
+// Numbers the push whose status is about to be published (false: no push ran).
+bool next_status(cpic_context* c) {
+  if (c->D == 0 || c->np == 0) return false;
+  ++c->push_seq;
+  c->push_pending = true;
+  return true;
+}
+
+int publish_status(cpic_context* c) {
+  if (!next_status(c)) return CPIC_OK;
+  k_publish_push<<<1, kBlock, 0, c->stream>>>(c->grp_rows, column_groups(c), c->err,
+                                              c->ovf_count, c->push_seq, c->push_host);
+  CHECK_LAUNCH();
+  return CPIC_OK;
+}
+
+// Waits for the status of the last push.  The device writes it while kernels
+// behind it are still queued; a stream that is done, or has failed, without
+// having written it ends the wait too.
+int await_status(cpic_context* c) {
+  auto written = [&] {
+    return __atomic_load_n(&c->push_host->seq, __ATOMIC_ACQUIRE) == c->push_seq;
+  };
+  while (!written()) {
+    for (int k = 0; k < 4096 && !written(); ++k) __builtin_ia32_pause();
+    if (written()) break;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    HIP_TRY(e);
+    if (!written()) return fail(CPIC_ERR_HIP, "the last push left no status");
   }
-  // error flags and max_count, the first and second status lines
-  HIP_TRY(hipMemcpyAsync(c->occ_host, c->status, (kStatusStride + 1) * sizeof(int),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipEventRecord(c->occ_event, c->stream));
-  c->occ_pending = true;
   return CPIC_OK;
 }
 
@@ -660,13 +742,13 @@ int regrow_columns(cpic_context* c, int D) {
 }
 
 int check_headroom(cpic_context* c) {
-  if (!c->occ_pending) return CPIC_OK;
-  HIP_TRY(hipEventSynchronize(c->occ_event));
-  c->occ_pending = false;
-  if (c->occ_host[0])
+  if (!c->push_pending) return CPIC_OK;
+  if (int s = await_status(c)) return s;
+  c->push_pending = false;
+  if (c->push_host->err)
     return fail(CPIC_ERR_DEVICE, "an earlier push failed on the device (flags=%d)",
-                c->occ_host[0]);
-  const int max_count = c->occ_host[kStatusStride];
+                c->push_host->err);
+  const int max_count = c->push_host->rows;
   if (c->D == 0 || max_count < c->D - std::max(8, c->D / 4)) return CPIC_OK;
   const int D = (c->D * 3 / 2 + 63) / 64 * 64;  // 1.5x the rows
   return with_real(c, [&](auto r) { return regrow_columns<decltype(r)>(c, D); });
@@ -786,6 +868,35 @@ int snapshot_wait(cpic_context* c, int slot, cpic_snapshot* out) {
 
 namespace {
 
+// The field stages of one step (unload, advance_b, advance_e, advance_b, and,
+// with erow >= 0, the energy partials into set erow) in three launches.
+template <class R>
+int stage_fields(cpic_context* c, const cpic_step_params* sp, int erow) {
+  const R px = (R)sp->px, py = (R)sp->py, pz = (R)sp->pz;
+  const R half = (R)0.5;
+  const R hpx = half * px, hpy = half * py, hpz = half * pz;
+  R cx, cy, cz;
+  unload_scales<R>((R)sp->dx, (R)sp->dy, (R)sp->dz, (R)sp->dt, cx, cy, cz);
+  const int blocks = cdiv(c->nc, kBlock);
+  R* fields = (R*)c->fields;
+  next_status(c);
+  k_current_advance_b<R><<<blocks + 1, kBlock, 0, c->stream>>>(
+      fields, (const R*)c->acc, c->grid, cx, cy, cz, hpx, hpy, hpz, c->grp_rows,
+      column_groups(c), c->err, c->ovf_count, c->push_seq, c->push_host);
+  CHECK_LAUNCH();
+  const long n = (c->nx + 1) * (c->ny + 1) * (c->nz + 1);
+  k_advance_e<R><<<cdiv(n, kBlock), kBlock, 0, c->stream>>>(fields, c->grid, px, py, pz,
+                                                            (R)sp->dt_eps0);
+  CHECK_LAUNCH();
+  if (erow >= 0)
+    k_advance_b_energy<R><<<blocks, kBlock, 0, c->stream>>>(
+        fields, c->grid, hpx, hpy, hpz, c->partials + 2 * (size_t)blocks * erow);
+  else
+    k_advance_b<R><<<blocks, kBlock, 0, c->stream>>>(fields, c->grid, hpx, hpy, hpz);
+  CHECK_LAUNCH();
+  return CPIC_OK;
+}
+
 // nsteps iterations of the loop body of example/example.cpp:216-279 on the
 // context's stream, no host synchronisation; energies of step s (1-based)
 // into dhist row s - 1 (3 doubles: E, B, kinetic) when dhist is not null,
@@ -797,6 +908,13 @@ int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, doubl
   const R px = (R)sp->px, py = (R)sp->py, pz = (R)sp->pz;
   const R half = (R)0.5;
   const R hpx = half * px, hpy = half * py, hpz = half * pz;
+  // the field stages share launches unless one of them is being timed
+  const unsigned timed = (1u << CPIC_STAGE_UNLOAD) | (1u << CPIC_STAGE_ADVANCE_B) |
+                         (1u << CPIC_STAGE_ADVANCE_E) | (1u << CPIC_STAGE_ENERGY);
+  const bool fuse_fields =
+      c->solver == CPIC_FIELD_SOLVER_EM && !(c->timing & timed) && c->np > 0 && c->D > 0;
+  const int eblocks = cdiv(c->nc, kBlock);
+  int erows = 0;  // sets of energy partials waiting to be summed
   for (int64_t step = 1; step <= nsteps; ++step) {
     int t;
     // With particles resident, pass 1 gathers each cell's interpolator from
@@ -808,22 +926,33 @@ int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, doubl
     // needed while ghost accumulators may hold data
     if (!c->acc_ghosts_zero && (t = stage_clear<R>(c))) return t;
     if ((t = check_headroom(c))) return t;
-    const int ci = sp->compact_interval > 0 ? sp->compact_interval : kCompactInterval;
-    const int compact = (c->pushes++ % ci == 0) ? 1 : 0;
+    const bool compact = packs_now(c, sp->compact_interval);
     const int gather = !fused ? kGatherRead : step == nsteps ? kGatherStore : kGatherFields;
     if ((t = stage_push<R>(c, (R)sp->qdt_2mc, (R)sp->cdt_dx, (R)sp->cdt_dy, (R)sp->cdt_dz,
                            (R)sp->qsp, 0, compact, gather)))
       return t;
-    if ((t = note_occupancy(c))) return t;
-    if ((t = stage_unload<R>(c, (R)sp->dx, (R)sp->dy, (R)sp->dz, (R)sp->dt))) return t;
-    if ((t = stage_advance_b<R>(c, hpx, hpy, hpz))) return t;
-    if ((t = stage_advance_e<R>(c, px, py, pz, (R)sp->dt_eps0))) return t;
-    if ((t = stage_advance_b<R>(c, hpx, hpy, hpz))) return t;
     const bool do_e = ei > 0 && step % ei == 0, do_k = ki > 0 && step % ki == 0;
-    if (do_e || do_k) {
+    double* row = dhist ? dhist + 3 * (step - 1) : c->red_out;
+    if (fuse_fields) {
+      if ((t = stage_fields<R>(c, sp, do_e ? erows : -1))) return t;
+      // the partials of many steps are summed by one launch (without a
+      // history, each step's into the same place: the last energies are kept)
+      if (do_e && (++erows == (dhist ? c->partial_rows : 1) || step + ei > nsteps)) {
+        if ((t = launch_energy_rows(c, erows, eblocks, row - (dhist ? 3 * ei * (erows - 1) : 0),
+                                    3 * ei)))
+          return t;
+        erows = 0;
+      }
+    } else {
+      if ((t = publish_status(c))) return t;
+      if ((t = stage_unload<R>(c, (R)sp->dx, (R)sp->dy, (R)sp->dz, (R)sp->dt))) return t;
+      if ((t = stage_advance_b<R>(c, hpx, hpy, hpz))) return t;
+      if ((t = stage_advance_e<R>(c, px, py, pz, (R)sp->dt_eps0))) return t;
+      if ((t = stage_advance_b<R>(c, hpx, hpy, hpz))) return t;
+    }
+    if ((do_e && !fuse_fields) || do_k) {
       StageTimer tm(c, CPIC_STAGE_ENERGY);
-      double* row = dhist ? dhist + 3 * (step - 1) : c->red_out;
-      if (do_e && (t = launch_field_energy<R>(c, row))) return t;
+      if (do_e && !fuse_fields && (t = launch_field_energy<R>(c, row))) return t;
       if (do_k && (t = launch_kinetic<R>(c, (double)sp->me * sp->c * sp->c, row + 2))) return t;
       if ((t = tm.finish())) return t;
     }
@@ -880,7 +1009,10 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
     c->cg.nc = (int)c->nc;
     c->cg.sy = (int)X;
     c->cg.sz = (int)(X * Y);
-    c->n_partials = 4096;
+    // one block's partial per kBlock cells (voxels for the ES energy), and as
+    // many steps' sets as 4 MB hold, 64 at most
+    c->n_partials = cdiv(c->ncells, kBlock);
+    c->partial_rows = std::clamp((int)((4L << 20) / (16L * c->n_partials)), 1, 64);
   
     auto bail = [&](int s) {
       cpic_destroy(c);
@@ -893,13 +1025,20 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
     if ((s = alloc(&c->fields, c->rsz() * 9 * c->ncells))) return bail(s);
     if ((s = alloc(&c->interp, c->rsz() * kInterpStride * c->ncells))) return bail(s);
     if ((s = alloc(&c->acc, c->rsz() * 12 * c->ncells))) return bail(s);
-    if ((s = alloc((void**)&c->partials, sizeof(double) * 3 * c->n_partials))) return bail(s);
+    if ((s = alloc((void**)&c->partials,
+                   sizeof(double) * (2 * (size_t)c->partial_rows + 1) * c->n_partials)))
+      return bail(s);
     if ((s = alloc((void**)&c->red_out, sizeof(double) * 4))) return bail(s);
-    if ((s = alloc((void**)&c->status, 4 * kStatusStride * sizeof(int)))) return bail(s);
+    if ((s = alloc((void**)&c->status, 3 * kStatusStride * sizeof(int)))) return bail(s);
     c->err = c->status;
-    c->max_count = c->status + kStatusStride;
-    c->movers = reinterpret_cast<unsigned int*>(c->status + 2 * kStatusStride);
-    c->ovf_count = reinterpret_cast<unsigned int*>(c->status + 3 * kStatusStride);
+    c->movers = reinterpret_cast<unsigned int*>(c->status + kStatusStride);
+    c->ovf_count = reinterpret_cast<unsigned int*>(c->status + 2 * kStatusStride);
+    if (hipHostMalloc((void**)&c->push_host, sizeof(PushStatus), hipHostMallocDefault) !=
+        hipSuccess) {
+      c->push_host = nullptr;
+      return bail(fail(CPIC_ERR_HIP, "pinned allocation failed"));
+    }
+    *c->push_host = PushStatus{};
     s = with_real(c, [&](auto r) {
       using R = decltype(r);
       int t;
@@ -909,7 +1048,7 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
       return CPIC_OK;
     });
     if (s) return bail(s);
-    if (hipMemsetAsync(c->status, 0, 4 * kStatusStride * sizeof(int), c->stream) != hipSuccess ||
+    if (hipMemsetAsync(c->status, 0, 3 * kStatusStride * sizeof(int), c->stream) != hipSuccess ||
         hipMemsetAsync(c->red_out, 0, sizeof(double) * 4, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return bail(fail(CPIC_ERR_HIP, "context initialisation failed"));
@@ -933,8 +1072,7 @@ int cpic_destroy(cpic_context* c) {
                     c->red_out, c->hist_dev,   c->gauss_q,  c->gauss_base, c->gauss_out};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
-    if (c->occ_event) (void)hipEventDestroy(c->occ_event);
-    if (c->occ_host) (void)hipHostFree(c->occ_host);
+    if (c->push_host) (void)hipHostFree(c->push_host);
     if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
     for (auto& sn : c->snap) free_snapshot(sn);
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
@@ -1062,14 +1200,16 @@ int upload_particles(cpic_context* c, int64_t n, const void* x, const void* y, c
         c->cnt[0], c->mask[0], (int)c->nc, (int)c->nc_pad, c->MW);
     CHECK_LAUNCH();
     // a fresh particle state: earlier device errors no longer apply
+    // (nor an overflow list that a failed push may have left)
     if ((t = fill_zero<int>(c, c->err, 1))) return t;
+    if ((t = fill_zero<unsigned int>(c, c->ovf_count, 1))) return t;
     HIP_TRY(hipStreamSynchronize(c->stream));
     return CPIC_OK;
   });
   if (s) return s;
   c->cur = 0;
   c->pushes = 0;
-  c->occ_pending = false;
+  c->push_pending = false;
   c->np = n;
   return CPIC_OK;
 }
@@ -1296,12 +1436,10 @@ int cpic_push(cpic_context* c, double qdt_2mc, double cdt_dx, double cdt_dy, dou
     return with_real(c, [&](auto r) {
       using R = decltype(r);
       if (int t = check_headroom(c)) return t;
-      // the first push after an upload and then every kCompactInterval-th one
-      // pack the columns
-      const int compact = (c->pushes++ % kCompactInterval == 0) ? 1 : 0;
+      const bool compact = packs_now(c, 0);
       if (int t = stage_push<R>(c, (R)qdt_2mc, (R)cdt_dx, (R)cdt_dy, (R)cdt_dz, (R)qsp, 1, compact))
         return t;
-      return note_occupancy(c);
+      return publish_status(c);
     });
   });
 }
@@ -1564,10 +1702,17 @@ int cpic_stage_times(cpic_context* c, int64_t* counts, double* ms) {
 int cpic_last_push_movers(cpic_context* c, int64_t* movers) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
+    // a tangent push counts in one word, a column push per group
     unsigned int m = 0;
+    std::vector<int> per(c->D > 0 && c->np > 0 ? (size_t)column_groups(c) : 0);
     HIP_TRY(hipMemcpyAsync(&m, c->movers, sizeof m, hipMemcpyDeviceToHost, c->stream));
+    if (!per.empty())
+      HIP_TRY(hipMemcpyAsync(per.data(), c->grp_movers, sizeof(int) * per.size(),
+                             hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (movers) *movers = m;
+    int64_t sum = m;
+    for (int k : per) sum += k;
+    if (movers) *movers = sum;
     return CPIC_OK;
   });
 }

@@ -295,13 +295,9 @@ __device__ __forceinline__ void for_each_ghost_image(const Grid& g, int x, int y
 // each thread also writes its voxel's new B into the ghosts it is the source
 // of (no thread reads B ghosts here).
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_advance_b(R* __restrict__ fields, Grid g, R px, R py, R pz) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= g.nx * g.ny * g.nz) return;
-  const int x = 1 + t % g.nx;
-  const int y = 1 + (t / g.nx) % g.ny;
-  const int z = 1 + t / (g.nx * g.ny);
-  const int i = voxel(g, x, y, z);
+__device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Grid& g, int x,
+                                                int y, int z, int i, R px, R py, R pz,
+                                                double* v = nullptr) {
   const size_t N = g.ncells;
   const R* ex = fields;
   const R* ey = fields + N;
@@ -316,11 +312,26 @@ __global__ void __launch_bounds__(kBlock) k_advance_b(R* __restrict__ fields, Gr
   bx[i] = nbx;
   by[i] = nby;
   bz[i] = nbz;
-  for_each_ghost_image(g, x, y, z, [&](int v) {
-    bx[v] = nbx;
-    by[v] = nby;
-    bz[v] = nbz;
+  for_each_ghost_image(g, x, y, z, [&](int w) {
+    bx[w] = nbx;
+    by[w] = nby;
+    bz[w] = nbz;
   });
+  if (v) {
+    const double e0 = e_x, e1 = e_y, e2 = e_z, b0 = nbx, b1 = nby, b2 = nbz;
+    v[0] = e0 * e0 + e1 * e1 + e2 * e2;
+    v[1] = b0 * b0 + b1 * b1 + b2 * b2;
+  }
+}
+
+template <class R>
+__global__ void __launch_bounds__(kBlock) k_advance_b(R* __restrict__ fields, Grid g, R px, R py, R pz) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= g.nx * g.ny * g.nz) return;
+  const int x = 1 + t % g.nx;
+  const int y = 1 + (t / g.nx) % g.ny;
+  const int z = 1 + t / (g.nx * g.ny);
+  advance_b_voxel(fields, g, x, y, z, voxel(g, x, y, z), px, py, pz);
 }
 
 // EM_Field_Solver::advance_e (src/fields.h:618-665), cells [1,n+1]^3, after
@@ -393,6 +404,24 @@ __device__ __forceinline__ void block_sum_store(double (&v)[NQ], double* out) {
       out[q] = s;
     }
   }
+}
+
+// advance_b and the energies of the fields it leaves, as k_advance_b followed
+// by k_field_energy_partial with one block per kBlock cells (the same sums in
+// the same order).
+template <class R>
+__global__ void __launch_bounds__(kBlock)
+k_advance_b_energy(R* __restrict__ fields, Grid g, R px, R py, R pz,
+                   double* __restrict__ partials) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  double v[2] = {0, 0};
+  if (t < g.nx * g.ny * g.nz) {
+    const int x = 1 + t % g.nx;
+    const int y = 1 + (t / g.nx) % g.ny;
+    const int z = 1 + t / (g.nx * g.ny);
+    advance_b_voxel(fields, g, x, y, z, voxel(g, x, y, z), px, py, pz, v);
+  }
+  block_sum_store<2>(v, partials + 2 * (size_t)blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -480,11 +509,15 @@ k_field_energy_partial(const R* __restrict__ fields, Grid g, double* __restrict_
   block_sum_store<2>(v, partials + 2 * blockIdx.x);
 }
 
-// Final pass: out[q] = scale[q] * sum_b partials[b][q], in block order.
+// Final pass: out[q] = scale[q] * sum_b partials[b][q], in block order.  Block
+// r of the grid does so for the r-th set of nblocks partials, into out +
+// r * out_stride.
 template <int NQ>
 __global__ void __launch_bounds__(kBlock)
 k_reduce_final(const double* __restrict__ partials, int nblocks, double s0, double s1,
-               double* __restrict__ out) {
+               double* __restrict__ out, int out_stride = 0) {
+  partials += (size_t)blockIdx.x * nblocks * NQ;
+  out += (size_t)blockIdx.x * out_stride;
   double v[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) v[q] = 0;

@@ -524,8 +524,12 @@ template <class R> struct PushPass {
   R qdt_2mc, cdt_dx, cdt_dy, cdt_dz, qsp;
   int accumulate;  // 1: acc += (push semantics), 0: acc = (after a clear)
   int* err;
-  unsigned* movers;
-  int* max_count;
+  // per group, written by pass 1: rows its columns use, and particles that
+  // took the move_p branch.  One plain store each: an atomic per wave on a
+  // shared counter took longer than the pass itself on small grids (32^3
+  // cells, 2048 waves: 45 us with the atomics)
+  int* grp_rows;
+  int* grp_movers;
 };
 
 // The interpolator of voxel v for pass 1: read from the array, or gathered
@@ -553,6 +557,61 @@ __device__ __forceinline__ void cell_interpolator(const PushPass<R>& a, int v, V
   }
 }
 
+// The push of one particle and its first streak (src/push.h:124-256): (pa, pb)
+// is its slot, (o0, o1) receives what its row of the output holds afterwards,
+// o its 12 contributions to the cell's accumulators.  Returns whether it took the move_p branch; d is the face
+// it left through, or -1 when it ends in its cell.  A particle that leaves
+// is stored with its position before the push.
+template <class R, class V4>
+__device__ __forceinline__ bool push_particle(const PushPass<R>& a, const V4& e0, const V4& e1,
+                                              const V4& e2, const V4& b0, const V4& b1,
+                                              const V4& pa, const V4& pb, R o[12], V4& o0,
+                                              V4& o1, int& d) {
+  const R one = 1.;
+  const R one_third = 1. / 3.;
+  const R dx = pa.x, dy = pa.y, dz = pa.z;
+  R ux = pa.w, uy = pb.x, uz = pb.y;
+  const R w = pb.z;
+  boris(e0, e1, e2, b0, b1, a.qdt_2mc, dx, dy, dz, ux, uy, uz);
+  // displacement in cell units, push.h:169-182
+  R ddx, ddy, ddz;
+  displacement(ux, uy, uz, a.cdt_dx, a.cdt_dy, a.cdt_dz, ddx, ddy, ddz);
+  const R mx = dx + ddx, my = dy + ddy, mz = dz + ddz;
+  const R nx = mx + ddx, ny = my + ddy, nz = mz + ddz;
+  const R q = w * a.qsp;
+  R px, py, pz;
+  d = -1;
+  // the deposit's inputs: the whole move (it stays in the cell,
+  // push.h:218-232) or the first streak of move_p
+  R s0 = ddx, s1 = ddy, s2 = ddz, m0 = mx, m1 = my, m2 = mz, v5;
+  const bool stays =
+      nx <= one && ny <= one && nz <= one && -nx <= one && -ny <= one && -nz <= one;
+  if (stays) {
+    v5 = q * ddx * ddy * ddz * one_third;
+    px = nx;
+    py = ny;
+    pz = nz;
+  } else {
+    R pos[3] = {dx, dy, dz};
+    R rem[3] = {ddx, ddy, ddz};
+    R dsp[3], mid[3];
+    d = streak_geometry(pos, rem, q, dsp, mid, v5);
+    s0 = dsp[0];
+    s1 = dsp[1];
+    s2 = dsp[2];
+    m0 = mid[0];
+    m1 = mid[1];
+    m2 = mid[2];
+    px = d < 0 ? pos[0] : dx;
+    py = d < 0 ? pos[1] : dy;
+    pz = d < 0 ? pos[2] : dz;
+  }
+  streak_values(q, s0, s1, s2, m0, m1, m2, v5, o);
+  o0.x = px; o0.y = py; o0.z = pz; o0.w = ux;
+  o1.x = uy; o1.y = uz; o1.z = w;  o1.w = pb.w;
+  return !stays;
+}
+
 // Pass 1: push + first streak, one lane per cell (src/push.h:65-295).
 // A particle that stays is stored with its new position.  A particle that
 // leaves through face d (after depositing its first streak here) is stored
@@ -572,9 +631,6 @@ __global__ void __launch_bounds__(kBlock) k_push_pass(PushPass<R> a) {
   typedef typename Vec4T<R>::type V4;
   V4 e0 = {}, e1 = {}, e2 = {}, b0 = {}, b1 = {};
   if (valid) cell_interpolator(a, v, e0, e1, e2, b0, b1);
-  const R one = 1.;
-  const R one_third = 1. / 3.;
-  const R qdt_2mc = a.qdt_2mc;
   LaneAcc<R, K> acc;
   acc.zero();
   int ns = 0, nmov = 0;
@@ -597,49 +653,11 @@ __global__ void __launch_bounds__(kBlock) k_push_pass(PushPass<R> a) {
 
   auto process = [&](bool have, const V4& pa, const V4& pb) {
     if (have) {
-      const R dx = pa.x, dy = pa.y, dz = pa.z;
-      R ux = pa.w, uy = pb.x, uz = pb.y;
-      const R w = pb.z;
-      boris(e0, e1, e2, b0, b1, qdt_2mc, dx, dy, dz, ux, uy, uz);
-      // displacement in cell units, push.h:169-182
-      R ddx, ddy, ddz;
-      displacement(ux, uy, uz, a.cdt_dx, a.cdt_dy, a.cdt_dz, ddx, ddy, ddz);
-      const R mx = dx + ddx, my = dy + ddy, mz = dz + ddz;
-      const R nx = mx + ddx, ny = my + ddy, nz = mz + ddz;
-      const R q = w * a.qsp;
-      R px, py, pz;
-      int d = -1;
-      // the deposit's inputs: the whole move (it stays in the cell,
-      // push.h:218-232) or the first streak of move_p
-      R s0 = ddx, s1 = ddy, s2 = ddz, m0 = mx, m1 = my, m2 = mz, v5;
-      if (nx <= one && ny <= one && nz <= one && -nx <= one && -ny <= one && -nz <= one) {
-        v5 = q * ddx * ddy * ddz * one_third;
-        px = nx;
-        py = ny;
-        pz = nz;
-      } else {
-        ++nmov;
-        R pos[3] = {dx, dy, dz};
-        R rem[3] = {ddx, ddy, ddz};
-        R dsp[3], mid[3];
-        d = streak_geometry(pos, rem, q, dsp, mid, v5);
-        s0 = dsp[0];
-        s1 = dsp[1];
-        s2 = dsp[2];
-        m0 = mid[0];
-        m1 = mid[1];
-        m2 = mid[2];
-        // a particle that leaves is stored with its position before the push
-        px = d < 0 ? pos[0] : dx;
-        py = d < 0 ? pos[1] : dy;
-        pz = d < 0 ? pos[2] : dz;
-      }
-      {
-        R o[12];
-        streak_values(q, s0, s1, s2, m0, m1, m2, v5, o);
-#pragma unroll
-        for (int k = 0; k < 12; ++k) acc.add(k, o[k]);
-      }
+      int d;
+      V4 o0, o1;
+      R o[12];
+      if (push_particle(a, e0, e1, e2, b0, b1, pa, pb, o, o0, o1, d)) ++nmov;
+      add12(acc, o);
       const int row = ns++;
       if ((row >> 6) != cw) {
         flush_dep();
@@ -654,7 +672,9 @@ __global__ void __launch_bounds__(kBlock) k_push_pass(PushPass<R> a) {
         dw4 |= d == 4 ? bit : 0ull;
         dw5 |= d == 5 ? bit : 0ull;
       }
-      store_particle(a.cs, ci, row, px, py, pz, ux, uy, uz, w, pb.w);
+      V4* dst = reinterpret_cast<V4*>(a.cs.out + col_slot(ci, row, a.cs.D) * kSlotLen);
+      dst[0] = o0;
+      dst[1] = o1;
     }
   };
 
@@ -714,8 +734,8 @@ __global__ void __launch_bounds__(kBlock) k_push_pass(PushPass<R> a) {
   a.cs.cnt_out[ci] = ns;
   const int wm = wave_sum_int(nmov);
   if ((threadIdx.x & 63) == 0) {
-    if (wm) atomicAdd(a.movers, (unsigned)wm);
-    atomicMax(a.max_count, lmax);
+    a.grp_movers[ci >> 6] = wm;
+    a.grp_rows[ci >> 6] = lmax;
     a.dep_words[ci >> 6] = (lmax + 63) >> 6;
   }
 }
@@ -860,190 +880,11 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
   }
 }
 
-// Pass 1 in place (every step but the compacting ones).  Same arithmetic as
-// k_push_pass; the memory pipeline differs.  Every row issues the same loads
-// and stores on every lane: a lane without a particle in the row stores
-// whatever it loaded when another lane of its 128-byte line holds one (the
-// row is free in the output column, and arrivals overwrite it later), and
-// otherwise its store is dropped by the buffer descriptor's range check.
-// The loads of row j + 1 are issued before the stores of row j, and with a
-// fixed number of instructions in between, the wait for them does not wait
-// for those stores.
-template <class R, bool K>
-__global__ void __launch_bounds__(kBlock) k_push_rows(PushPass<R> a) {
-  if (__builtin_amdgcn_readfirstlane(*a.err)) return;  // an earlier push failed
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;  // < nc_pad
-  const bool valid = ci < a.g.nc;
-  const int len = valid ? min(a.cs.cnt_in[ci], a.cs.D) : 0;
-  // rows walked: the longest column of the wave, rounded up to even so that
-  // both rows of every loop iteration are processed (D is a multiple of 8,
-  // so the extra row is a row past every column's end)
-  const int lreal = wave_max_int(len);
-  const int lmax = (lreal + 1) & ~1;
-  const int v = valid ? interior_to_voxel(a.g, ci) : 0;
-  typedef typename Vec4T<R>::type V4;
-  V4 e0 = {}, e1 = {}, e2 = {}, b0 = {}, b1 = {};
-  if (valid) cell_interpolator(a, v, e0, e1, e2, b0, b1);
-  const R one = 1.;
-  const R one_third = 1. / 3.;
-  const R qdt_2mc = a.qdt_2mc;
-  LaneAcc<R, K> acc;
-  acc.zero();
-  int hi = 0, nmov = 0;
-  unsigned long long m_in = 0, m_out = 0;
-  unsigned long long dw0 = 0, dw1 = 0, dw2 = 0, dw3 = 0, dw4 = 0, dw5 = 0;
-  const size_t MP = a.cs.nc_pad;
-  const int MW = a.cs.MW;
-  const R* const dummy = a.cs.in;
-  // Row stores go through a buffer descriptor over the wave's column group:
-  // a store at an offset past its end is dropped without a branch.  A lane
-  // stores whenever a lane of its 128-byte line of the row holds a particle
-  // (a free row receives whatever was loaded), so memory only ever sees whole
-  // lines (a partly written line costs a read-modify-write), and rows past
-  // the ends of all the columns of a line cost nothing.
-  const int lane = threadIdx.x & 63;
-  const int grp = __builtin_amdgcn_readfirstlane(ci >> 6);
-  const int gbytes = a.cs.D * 64 * kSlotLen * (int)sizeof(R);
-  const __amdgpu_buffer_rsrc_t rows_out = __builtin_amdgcn_make_buffer_rsrc(
-      a.cs.out + (size_t)grp * a.cs.D * 64 * kSlotLen, 0, gbytes, kBufferWord3);
-  constexpr int kLine = 128 / (kSlotLen * (int)sizeof(R));  // lanes per line
-  static_assert(kLine >= 1 && kLine < 64 && (kLine & (kLine - 1)) == 0, "line of slots");
-  const int line0 = lane & ~(kLine - 1);
-
-  // loads of row r into (x, y); returns whether the row holds a particle
-  auto request = [&](int r, V4& x, V4& y) -> bool {
-    if ((r & 63) == 0) {
-      m_in = (valid && r < len) ? a.cs.mask_in[(size_t)(r >> 6) * MP + ci] : 0ull;
-      settle(m_in);  // once per 64 rows
-    }
-    const bool ok = valid && r < len && ((m_in >> (r & 63)) & 1ull);
-    const V4* src = reinterpret_cast<const V4*>(ok ? a.cs.in + col_slot(ci, r, a.cs.D) * kSlotLen
-                                                   : dummy);
-    x = src[0];
-    y = src[1];
-    return ok;
-  };
-
-  auto process = [&](int j, bool have, const V4& pa, const V4& pb) {
-    const int b = j & 63;
-    V4 o0 = pa, o1 = pb;  // what row j of the output receives
-    if (have) {
-      const R dx = pa.x, dy = pa.y, dz = pa.z;
-      R ux = pa.w, uy = pb.x, uz = pb.y;
-      const R w = pb.z;
-      boris(e0, e1, e2, b0, b1, qdt_2mc, dx, dy, dz, ux, uy, uz);
-      R ddx, ddy, ddz;
-      displacement(ux, uy, uz, a.cdt_dx, a.cdt_dy, a.cdt_dz, ddx, ddy, ddz);
-      const R mx = dx + ddx, my = dy + ddy, mz = dz + ddz;
-      const R nx = mx + ddx, ny = my + ddy, nz = mz + ddz;
-      const R q = w * a.qsp;
-      R px, py, pz;
-      // the deposit's inputs: the whole move (it stays in the cell,
-      // push.h:218-232) or the first streak of move_p
-      R s0 = ddx, s1 = ddy, s2 = ddz, m0 = mx, m1 = my, m2 = mz, v5;
-      if (nx <= one && ny <= one && nz <= one && -nx <= one && -ny <= one && -nz <= one) {
-        v5 = q * ddx * ddy * ddz * one_third;
-        px = nx;
-        py = ny;
-        pz = nz;
-      } else {
-        ++nmov;
-        R pos[3] = {dx, dy, dz};
-        R rem[3] = {ddx, ddy, ddz};
-        R dsp[3], mid[3];
-        const int d = streak_geometry(pos, rem, q, dsp, mid, v5);
-        s0 = dsp[0];
-        s1 = dsp[1];
-        s2 = dsp[2];
-        m0 = mid[0];
-        m1 = mid[1];
-        m2 = mid[2];
-        // a particle that leaves is stored with its position before the push
-        px = d < 0 ? pos[0] : dx;
-        py = d < 0 ? pos[1] : dy;
-        pz = d < 0 ? pos[2] : dz;
-        const unsigned long long bit = 1ull << b;
-        dw0 |= d == 0 ? bit : 0ull;
-        dw1 |= d == 1 ? bit : 0ull;
-        dw2 |= d == 2 ? bit : 0ull;
-        dw3 |= d == 3 ? bit : 0ull;
-        dw4 |= d == 4 ? bit : 0ull;
-        dw5 |= d == 5 ? bit : 0ull;
-      }
-      {
-        R o[12];
-        streak_values(q, s0, s1, s2, m0, m1, m2, v5, o);
-#pragma unroll
-        for (int k = 0; k < 12; ++k) acc.add(k, o[k]);
-      }
-      m_out |= 1ull << b;
-      hi = j + 1;
-      o0.x = px; o0.y = py; o0.z = pz; o0.w = ux;
-      o1.x = uy; o1.y = uz; o1.z = w;  o1.w = pb.w;
-    }
-    const unsigned long long occ = __ballot(have);
-    const bool st = (occ >> line0) & ((1ull << kLine) - 1);
-    const int off = st ? (j * 64 + lane) * kSlotLen * (int)sizeof(R) : gbytes;
-    store_slot(rows_out, off, o0, o1);
-    if (b == 63 || j == lmax - 1) {
-      const int wd = j >> 6;
-      a.cs.mask_out[(size_t)wd * MP + ci] = m_out;
-      a.dep[dep_index(0, wd, MW, MP, ci)] = dw0;
-      a.dep[dep_index(1, wd, MW, MP, ci)] = dw1;
-      a.dep[dep_index(2, wd, MW, MP, ci)] = dw2;
-      a.dep[dep_index(3, wd, MW, MP, ci)] = dw3;
-      a.dep[dep_index(4, wd, MW, MP, ci)] = dw4;
-      a.dep[dep_index(5, wd, MW, MP, ci)] = dw5;
-      a.dep[dep_index(6, wd, MW, MP, ci)] = dw0 | dw1 | dw2 | dw3 | dw4 | dw5;
-      m_out = dw0 = dw1 = dw2 = dw3 = dw4 = dw5 = 0;
-    }
-  };
-
-  // two row buffers in turn, one row ahead.  Each wait is preceded by the
-  // same instructions on every path into it (two loads and two stores after
-  // the awaited loads), so it waits for the awaited loads only; on entry,
-  // two stores of values rewritten at the end stand in for the stores of
-  // the previous row.
-  V4 xa = {}, ya = {}, xb = {}, yb = {};
-  bool ha = request(0, xa, ya);
-  bool hb = request(1, xb, yb);
-  a.cs.cnt_out[ci] = 0;
-  a.cs.mask_out[ci] = 0ull;
-  for (int j = 0; j < lmax; j += 2) {
-    settle(xa);
-    settle(ya);
-    process(j, ha, xa, ya);
-    ha = request(j + 2, xa, ya);
-    settle(xb);
-    settle(yb);
-    process(j + 1, hb, xb, yb);
-    hb = request(j + 3, xb, yb);
-  }
-
-  if (valid) {
-    const size_t N = a.ncells;
-    if (a.accumulate) {
-#pragma unroll
-      for (int k = 0; k < 12; ++k) a.acc[k * N + v] += acc.total(k);
-    } else {
-#pragma unroll
-      for (int k = 0; k < 12; ++k) a.acc[k * N + v] = acc.total(k);
-    }
-  }
-  for (int w = (lmax + 63) >> 6; w < MW; ++w) a.cs.mask_out[(size_t)w * MP + ci] = 0ull;
-  a.cs.cnt_out[ci] = hi;
-  const int wm = wave_sum_int(nmov);
-  if ((threadIdx.x & 63) == 0) {
-    if (wm) atomicAdd(a.movers, (unsigned)wm);
-    atomicMax(a.max_count, lreal);
-    a.dep_words[ci >> 6] = (lmax + 63) >> 6;
-  }
-}
-
 template <class R> struct ArrivePass {
   ColState<R> cs;                        // cs.out: the columns of pass 1
   const unsigned long long* dep;         // departure masks of pass 1
   const int* dep_words;                  // words of them written per group
+  unsigned long long* taken;             // [MW][nc_pad] scratch for columns deeper than LDS holds
   RecordList<R> out;                     // records of the next crossings
   Overflow<R> ovf;
   R* acc;
@@ -1053,166 +894,24 @@ template <class R> struct ArrivePass {
   int* err;
 };
 
-// Pass 2: every particle that left a cell in pass 1 continues in the cell
-// across the face it crossed.  The owner of that cell finds it through the
-// departure masks of its six neighbours, reads it from the neighbour's
-// column, recomputes its displacement and first streak (the same operations
-// as pass 1, without the deposit, which pass 1 made), and runs the next
-// streak.  Afterwards each cell releases the rows of its own departures.
-template <class R, bool K>
-__global__ void __launch_bounds__(kBlock) k_arrive_pass(ArrivePass<R> a) {
-  if (__builtin_amdgcn_readfirstlane(*a.err)) return;  // this push already failed
-  // groups in reverse order: the first blocks dispatched take the groups
-  // pass 1 wrote last, whose lines the 256 MB Infinity Cache still holds
-  // (14 us less than in pass 1's order), and the last ones end at the groups
-  // the next pass 1 starts with
-  const int ci = (gridDim.x - 1 - blockIdx.x) * blockDim.x + threadIdx.x;  // < nc_pad
-  const bool valid = ci < a.g.nc;
-  const size_t MP = a.cs.nc_pad;
-  const int MW = a.cs.MW;
-  const size_t NC = a.g.nc;
-  typedef typename Vec4T<R>::type V4;
-  // a particle that crossed face d came from the neighbour across the
-  // opposite face
-  int s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0;
-  int v = 0;
-  if (valid) {
-    int nb[6];
-    face_neighbors6(a.g, ci, nb, v);
-    s0 = nb[3];
-    s1 = nb[4];
-    s2 = nb[5];
-    s3 = nb[0];
-    s4 = nb[1];
-    s5 = nb[2];
-  }
-  RowCursor<R> rows;
-  {
-    const int l = valid ? min(a.cs.cnt_out[ci], a.cs.D) : 0;
-    unsigned long long w0 = valid ? a.cs.mask_out[ci] : 0ull;
-    settle(w0);
-    rows.start(l, w0);
-  }
-  LaneAcc<R, K> acc;
-  acc.zero();
-  int kd[6] = {0, 0, 0, 0, 0, 0};
-  int total_all = 0;
-  const R* dummy = a.cs.out;
-
-  // words of the departure masks to read: those pass 1 wrote for the
-  // source groups (usually one).  Pass 1 writes only the words of its
-  // group's rows, so a word at or past its group's count is no departure.
-  int nw = 0;
-  int ws0 = 0, ws1 = 0, ws2 = 0, ws3 = 0, ws4 = 0, ws5 = 0;
-  if (valid) {
-    ws0 = a.dep_words[s0 >> 6];
-    ws1 = a.dep_words[s1 >> 6];
-    ws2 = a.dep_words[s2 >> 6];
-    ws3 = a.dep_words[s3 >> 6];
-    ws4 = a.dep_words[s4 >> 6];
-    ws5 = a.dep_words[s5 >> 6];
-    nw = max(max(ws0, ws1), max(max(ws2, ws3), max(ws4, ws5)));
-  }
-  nw = min(wave_max_int(nw), MW);
-  for (int w = 0; w < nw; ++w) {
-    unsigned long long d0 = 0, d1 = 0, d2 = 0, d3 = 0, d4 = 0, d5 = 0;
-    if (valid) {
-      if (w < ws0) d0 = a.dep[dep_index(0, w, MW, MP, s0)];
-      if (w < ws1) d1 = a.dep[dep_index(1, w, MW, MP, s1)];
-      if (w < ws2) d2 = a.dep[dep_index(2, w, MW, MP, s2)];
-      if (w < ws3) d3 = a.dep[dep_index(3, w, MW, MP, s3)];
-      if (w < ws4) d4 = a.dep[dep_index(4, w, MW, MP, s4)];
-      if (w < ws5) d5 = a.dep[dep_index(5, w, MW, MP, s5)];
-    }
-    const int total = __popcll(d0) + __popcll(d1) + __popcll(d2) + __popcll(d3) +
-                      __popcll(d4) + __popcll(d5);
-    total_all += total;
-    const int tmax = wave_max_int(total);
-    if (tmax == 0) continue;
-    // the next departure to read: face d, bits left in the current word
-    int d = 0;
-    unsigned long long bits = d0;
-    auto request = [&](int i, V4& x, V4& y) {
-      const R* src = dummy;
-      if (i < total) {
-        while (bits == 0 && d < 5) {
-          ++d;
-          bits = d == 1 ? d1 : d == 2 ? d2 : d == 3 ? d3 : d == 4 ? d4 : d5;
-        }
-        if (bits != 0) {  // always, while the counts are consistent
-          const int r = 64 * w + __ffsll((long long)bits) - 1;
-          bits &= bits - 1;
-          const int sc = sel6(d, s0, s1, s2, s3, s4, s5);
-          src = a.cs.out + col_slot(sc, r, a.cs.D) * kSlotLen;
-        } else {
-          atomicOr(a.err, kErrBadCell);
-        }
-      }
-      const V4* p = reinterpret_cast<const V4*>(src);
-      x = p[0];
-      y = p[1];
-    };
-    auto process = [&](const V4& pa, const V4& pb) {
-      const R ux = pa.w, uy = pb.x, uz = pb.y, w8 = pb.z;
-      R pos[3] = {pa.x, pa.y, pa.z};
-      R rem[3];
-      displacement(ux, uy, uz, a.cdt_dx, a.cdt_dy, a.cdt_dz, rem[0], rem[1], rem[2]);
-      const R q = w8 * a.qsp;
-      // the first streak, deposited by the neighbour in pass 1: its
-      // geometry only
-      {
-        R dsp[3], mid[3], v5;
-        if (streak_geometry(pos, rem, q, dsp, mid, v5) < 0) atomicOr(a.err, kErrBadCell);
-      }
-      const int d2n = streak(pos, rem, q, acc);
-      if (d2n < 0) {
-        const int row = rows.next(a.cs, ci);
-        if (row >= 0)
-          store_particle(a.cs, ci, row, pos[0], pos[1], pos[2], ux, uy, uz, w8, pb.w);
-        else
-          atomicOr(a.err, kErrColumnFull);
-      } else {
-        int kk = kd[d2n];
-        put_record(a.out, a.ovf, a.g, ci, d2n, kk, pos, rem, ux, uy, uz, w8, pb.w, a.err);
-        kd[d2n] = kk;
-      }
-    };
-    for (int i0 = 0; i0 < tmax; i0 += kRecBatch) {
-      V4 x[kRecBatch], y[kRecBatch];
-#pragma unroll
-      for (int u = 0; u < kRecBatch; ++u) request(i0 + u, x[u], y[u]);
-#pragma unroll
-      for (int u = 0; u < kRecBatch; ++u) {
-        settle(x[u]);
-        settle(y[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kRecBatch; ++u)
-        if (i0 + u < total) process(x[u], y[u]);
-    }
-  }
-
-  if (valid) {
-    rows.finish(a.cs, ci);
-    a.cs.cnt_out[ci] = rows.len;
-    if (total_all > 0) {
-      const size_t N = a.ncells;
-#pragma unroll
-      for (int k = 0; k < 12; ++k) a.acc[k * N + v] += acc.total(k);
-    }
-    // release the rows of this cell's own departures: only their mask bits
-    // are cleared here.  Other lanes may still be reading those rows in this
-    // pass, but no lane writes them before the next pass, which is the first
-    // that can hand them out again.
-    const int own_words = min(a.dep_words[ci >> 6], MW);
-    for (int w = 0; w < own_words; ++w) {
-      const unsigned long long own = a.dep[dep_index(6, w, MW, MP, ci)];
-      if (own) a.cs.mask_out[(size_t)w * MP + ci] &= ~own;
-    }
-#pragma unroll
-    for (int dd = 0; dd < 6; ++dd)
-      a.out.cnt[(size_t)dd * NC + ci] = (unsigned char)min(kd[dd], a.out.M);
-  }
+// One arrival: the displacement and the first streak (whose deposit pass 1
+// made) recomputed from the stored slot (pa, pb), then the streak in the
+// calling lane's cell, whose 12 contributions o receives.  pos and rem receive
+// the state after it; returns the face crossed next, or -1 when the track
+// ends here.
+template <class R, class V4>
+__device__ __forceinline__ int arrive_particle(const ArrivePass<R>& a, const V4& pa, const V4& pb,
+                                               R o[12], R pos[3], R rem[3]) {
+  pos[0] = pa.x;
+  pos[1] = pa.y;
+  pos[2] = pa.z;
+  displacement(pa.w, pb.x, pb.y, a.cdt_dx, a.cdt_dy, a.cdt_dz, rem[0], rem[1], rem[2]);
+  const R q = pb.z * a.qsp;
+  R dsp[3], mid[3], v5;
+  if (streak_geometry(pos, rem, q, dsp, mid, v5) < 0) atomicOr(a.err, kErrBadCell);
+  const int d = streak_geometry(pos, rem, q, dsp, mid, v5);
+  streak_values(q, dsp[0], dsp[1], dsp[2], mid[0], mid[1], mid[2], v5, o);
+  return d;
 }
 
 // Fallback for spilled records: one thread per record walks the particle to
@@ -1276,6 +975,89 @@ __global__ void __launch_bounds__(kBlock) k_spill_pass(SpillPass<R> a) {
       atomicOr(a.err, kErrColumnFull);
     }
   }
+}
+
+// What the host wants to know of a push before it launches the next one, in
+// pinned host memory that the device writes directly (a copy command and its
+// event cost the stream more than the smallest kernels of the step).
+struct PushStatus {
+  int err;    // device error flags
+  int rows;   // largest column occupancy (rows in use before the push)
+  int seq;    // number of the push, written last
+};
+
+// One block: the status of push seq to the host, and the overflow list's count
+// cleared for the next push.  Runs after every pass of the push.
+__device__ __forceinline__ void publish_push(const int* __restrict__ grp_rows, int ngroups,
+                                             const int* err, unsigned* ovf_count, int seq,
+                                             PushStatus* host) {
+  __shared__ int part[kBlock / 64];
+  int m = 0;
+  for (int i = threadIdx.x; i < ngroups; i += kBlock) m = max(m, grp_rows[i]);
+  m = wave_max_int(m);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int k = 1; k < kBlock / 64; ++k) m = max(m, part[k]);
+  *ovf_count = 0;
+  __hip_atomic_store(&host->err, *err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&host->rows, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void __launch_bounds__(kBlock)
+k_publish_push(const int* __restrict__ grp_rows, int ngroups, const int* err,
+               unsigned* ovf_count, int seq, PushStatus* host) {
+  publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
+}
+
+// The field stages between the push and advance_e in one launch (the fused
+// step's; small grids are bound by the number of launches): unload
+// (src/accumulator.cpp:45-122), the J fold (k_fold_j's closed form, from the
+// accumulators directly: a voxel of the high ghost layer is unloaded by the
+// thread whose voxel it folds into) and advance_b with its ghosts, in the
+// order of the separate kernels for every value.  J is written on interior
+// voxels only: k_advance_e, which follows, writes the ghosts.  The last block
+// has no cells and publishes the push's status.
+template <class R>
+__global__ void __launch_bounds__(kBlock)
+k_current_advance_b(R* __restrict__ fields, const R* __restrict__ acc, Grid g, R cx, R cy, R cz,
+                    R px, R py, R pz, const int* __restrict__ grp_rows, int ngroups,
+                    const int* err, unsigned* ovf_count, int seq, PushStatus* host) {
+  if (blockIdx.x == gridDim.x - 1) {
+    publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
+    return;
+  }
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= g.nx * g.ny * g.nz) return;
+  const int x = 1 + t % g.nx;
+  const int y = 1 + (t / g.nx) % g.ny;
+  const int z = 1 + t / (g.nx * g.ny);
+  const int i = voxel(g, x, y, z);
+  const size_t N = g.ncells;
+  const int pos[3] = {x, y, z};
+  const int n[3] = {g.nx, g.ny, g.nz};
+  const int st[3] = {1, g.sy, g.sz};
+  const R scale[3] = {cx, cy, cz};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const int ap = (c + 1) % 3, aq = (c + 2) % 3;
+    const int sp = st[ap], sq = st[aq];
+    const R* A = acc + (size_t)(4 * c) * N;
+    auto unloaded = [&](int v) {
+      return scale[c] * (A[v] + A[N + v - sp] + A[2 * N + v - sq] + A[3 * N + v - sp - sq]);
+    };
+    const int ip = i + n[ap] * sp, iq = i + n[aq] * sq;  // the images of faces p = 1, q = 1
+    R J = unloaded(i);
+    if (pos[ap] == 1 && pos[aq] == 1)
+      J = (J + unloaded(ip)) + (unloaded(iq) + unloaded(ip + n[aq] * sq));
+    else if (pos[ap] == 1)
+      J = J + unloaded(ip);
+    else if (pos[aq] == 1)
+      J = J + unloaded(iq);
+    fields[(6 + c) * N + i] = J;
+  }
+  advance_b_voxel(fields, g, x, y, z, i, px, py, pz);
 }
 
 // uncenter_particles, src/uncenter_p.h:4-105: for every particle, a
