@@ -243,3 +243,25 @@ def test_column_mode_gradient_equals_tangent():
     print(f"A_3 = {A:.6e}; dA_3/dB_z: adjoint {g_adj:.12e}, tangent {g_tan:.12e} (rel {rel:.2e}), "
           f"central differences {fd:.6e}")
     assert rel < 1e-8
+
+
+def test_gradient_is_the_same_with_buffers_in_place():
+    """A second gradient of the same shape reuses the first one's buffers,
+    one of another shape and back does not: the same bits each time."""
+    dtype = np.float32
+    st, _ = states.random_state(5, 4, 6, 4, dtype, seed=8)
+    k = dict(states.step_consts(dtype), energy_interval=1)
+    rng = np.random.default_rng(3)
+    sf = rng.standard_normal((9, st.fields.size // 9))
+    sp = rng.standard_normal((6, st.np))
+    out = []
+    with Simulation(st.nx, st.ny, st.nz, st.np, dtype) as sim, Adjoint(sim) as adj:
+        for steps, every, seeds in ((4, 2, sp), (4, 2, sp), (3, 1, None), (4, 2, sp), (5, 3, None)):
+            sim.upload_fields(st.fields)
+            sim.upload_particles(*[st.p[m] for m in ("x", "y", "z", "ux", "uy", "uz", "w")], st.cell)
+            hist = adj.forward(k, steps, every)
+            out.append((steps, hist, *adj.backward(sf, seeds)))
+    first = [o for o in out if o[0] == 4]
+    for o in first[1:]:
+        for a, b in zip(first[0][1:], o[1:]):
+            assert np.array_equal(a, b, equal_nan=True)
