@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/cabanapic_amd.h"
+#include "cpic_host_copy.h"
 #include "cpic_push_kernels.h"
 #include "cpic_split_kernels.h"
 #include "cpic_tangent_kernels.h"
@@ -988,6 +989,7 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
   
     cpic_context* c = new (std::nothrow) cpic_context();
     if (!c) return fail(CPIC_ERR_INVALID, "out of host memory");
+    HostRing::get().retain();
     c->real_size = cfg->real_size;
     c->nx = cfg->nx;
     c->ny = cfg->ny;
@@ -1078,6 +1080,7 @@ int cpic_destroy(cpic_context* c) {
     if (c->copy_stream) (void)hipStreamDestroy(c->copy_stream);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    HostRing::get().release();
     return CPIC_OK;
   });
 }
@@ -1263,16 +1266,11 @@ int download_particles(cpic_context* c, int64_t n, void* x, void* y, void* z, vo
     return CPIC_OK;
   });
   if (s) return s;
+  HostRing& ring = HostRing::get();
   for (int k = 0; k < 7; ++k)
-    if (dst[k])
-      HIP_TRY(hipMemcpyAsync(dst[k], soa + k * rs * n, rs * n, hipMemcpyDeviceToHost,
-                             c->stream));
-  if (cell)
-    HIP_TRY(hipMemcpyAsync(cell, cell_dev, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
-  if (tag)
-    HIP_TRY(hipMemcpyAsync(tag, tag_dev, sizeof(long long) * n, hipMemcpyDeviceToHost,
-                           c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+    if (dst[k]) HIP_TRY(ring.copy(dst[k], soa + k * rs * n, rs * n, c->stream));
+  if (cell) HIP_TRY(ring.copy(cell, cell_dev, sizeof(int) * n, c->stream));
+  if (tag) HIP_TRY(ring.copy(tag, tag_dev, sizeof(long long) * n, c->stream));
   return CPIC_OK;
 }
 
@@ -1342,8 +1340,7 @@ int cpic_download_fields(cpic_context* c, void* f) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
     if (!f) return fail(CPIC_ERR_INVALID, "null fields");
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    HIP_TRY(hipMemcpy(f, c->fields, c->rsz() * 9 * c->ncells, hipMemcpyDeviceToHost));
+    HIP_TRY(HostRing::get().copy(f, c->fields, c->rsz() * 9 * c->ncells, c->stream));
     return CPIC_OK;
   });
 }
