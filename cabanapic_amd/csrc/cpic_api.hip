@@ -133,9 +133,8 @@ struct cpic_context : ColumnSet {
   long pushes = 0;         // pushes since the last upload (the first of every
                            // compaction interval packs the columns)
   // device status words, one allocation (status), each on its own 256-byte
-  // line: [0] error flags (err), [kStatusStride] particles that left their
-  // cell in a tangent push (movers), [2 kStatusStride] overflow records
-  // (ovf_count, zero between pushes)
+  // line: [0] error flags (err), [kStatusStride] overflow records (ovf_count,
+  // zero between pushes)
   int* status = nullptr;
   unsigned int* ovf_count = nullptr;
 
@@ -148,7 +147,8 @@ struct cpic_context : ColumnSet {
   int partial_rows = 1;
   double* red_out = nullptr;   // [E, B, KE]
   int* err = nullptr;
-  unsigned int* movers = nullptr;
+  int* block_movers = nullptr;  // movers of the last tangent push, per block (not owned)
+  int n_block_movers = 0;
   double* hist_dev = nullptr;  // per-step energy rows of cpic_step
   long hist_cap = 0;           // rows allocated in hist_dev
   int n_partials = 0;
@@ -1031,10 +1031,9 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
                    sizeof(double) * (2 * (size_t)c->partial_rows + 1) * c->n_partials)))
       return bail(s);
     if ((s = alloc((void**)&c->red_out, sizeof(double) * 4))) return bail(s);
-    if ((s = alloc((void**)&c->status, 3 * kStatusStride * sizeof(int)))) return bail(s);
+    if ((s = alloc((void**)&c->status, 2 * kStatusStride * sizeof(int)))) return bail(s);
     c->err = c->status;
-    c->movers = reinterpret_cast<unsigned int*>(c->status + kStatusStride);
-    c->ovf_count = reinterpret_cast<unsigned int*>(c->status + 2 * kStatusStride);
+    c->ovf_count = reinterpret_cast<unsigned int*>(c->status + kStatusStride);
     if (hipHostMalloc((void**)&c->push_host, sizeof(PushStatus), hipHostMallocDefault) !=
         hipSuccess) {
       c->push_host = nullptr;
@@ -1050,7 +1049,7 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
       return CPIC_OK;
     });
     if (s) return bail(s);
-    if (hipMemsetAsync(c->status, 0, 3 * kStatusStride * sizeof(int), c->stream) != hipSuccess ||
+    if (hipMemsetAsync(c->status, 0, 2 * kStatusStride * sizeof(int), c->stream) != hipSuccess ||
         hipMemsetAsync(c->red_out, 0, sizeof(double) * 4, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return bail(fail(CPIC_ERR_HIP, "context initialisation failed"));
@@ -1699,15 +1698,15 @@ int cpic_stage_times(cpic_context* c, int64_t* counts, double* ms) {
 int cpic_last_push_movers(cpic_context* c, int64_t* movers) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
-    // a tangent push counts in one word, a column push per group
-    unsigned int m = 0;
-    std::vector<int> per(c->D > 0 && c->np > 0 ? (size_t)column_groups(c) : 0);
-    HIP_TRY(hipMemcpyAsync(&m, c->movers, sizeof m, hipMemcpyDeviceToHost, c->stream));
+    // counted per block by a tangent push, per group by a column push
+    const bool columns = c->D > 0 && c->np > 0;
+    const int* from = columns ? c->grp_movers : c->block_movers;
+    std::vector<int> per((size_t)(columns ? column_groups(c) : c->n_block_movers));
     if (!per.empty())
-      HIP_TRY(hipMemcpyAsync(per.data(), c->grp_movers, sizeof(int) * per.size(),
-                             hipMemcpyDeviceToHost, c->stream));
+      HIP_TRY(hipMemcpyAsync(per.data(), from, sizeof(int) * per.size(), hipMemcpyDeviceToHost,
+                             c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    int64_t sum = m;
+    int64_t sum = 0;
     for (int k : per) sum += k;
     if (movers) *movers = sum;
     return CPIC_OK;

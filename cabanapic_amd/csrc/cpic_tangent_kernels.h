@@ -94,7 +94,7 @@ template <class R> struct TangentPush {
   int ncells;               // Ng
   R qdt_2mc, cdt_dx, cdt_dy, cdt_dz, qsp;
   int* err;
-  unsigned* movers;
+  int* movers;              // [blocks] particles of the block that left their cell
 };
 
 // A block's accumulator window in LDS: kTanWindow consecutive voxels from
@@ -200,11 +200,12 @@ __device__ __forceinline__ void deposit_runs(const TangentPush<R>& a, const TanW
 }
 
 // The push of particle p (nothing for p >= n); returns the voxel of its own
-// cell, whose deposits are left in own[], or -1.
+// cell, whose deposits are left in own[], or -1.  left: whether it left that
+// cell.
 template <class R>
 __device__ __forceinline__ int push_tangent_particle(const TangentPush<R>& a,
                                                      const TanWindow<R>& win, int p,
-                                                     Dual<R> own[12]) {
+                                                     Dual<R> own[12], bool& left) {
   if (p >= a.n) return -1;
   typedef Dual<R> D;
   typedef typename Vec4T<R>::type V4;
@@ -261,11 +262,7 @@ __device__ __forceinline__ int push_tangent_particle(const TangentPush<R>& a,
     pos[1] = ny;
     pos[2] = nz;
   } else {
-    // one counter update per wave: the lowest active lane adds the number
-    // of lanes that leave their cell
-    const unsigned long long leaving = __ballot(1);
-    if ((threadIdx.x & 63) == (unsigned)__ffsll((long long)leaving) - 1)
-      atomicAdd(a.movers, (unsigned)__popcll(leaving));
+    left = true;
     pos[0] = dx;
     pos[1] = dy;
     pos[2] = dz;
@@ -380,6 +377,7 @@ k_push_tangent(TangentPush<R> a) {
   __shared__ double wt[12][kTanWindow];
   __shared__ R sv[12][4][kTanSide];
   __shared__ double st[12][4][kTanSide];
+  __shared__ int wmovers[kBlock / 64];
   const int p0 = blockIdx.x * blockDim.x;
   TanWindow<R> win{(p0 < a.n ? a.src_cell[p0] : 0) - 1, a.g.sy, a.g.sz, wv, wt, sv, st};
   for (int i = threadIdx.x; i < 12 * kTanWindow; i += blockDim.x) {
@@ -395,9 +393,21 @@ k_push_tangent(TangentPush<R> a) {
   D own[12];  // deposits into the particle's own cell
   // every lane takes part in the wave's run sums, so a lane without a
   // particle (or with an invalid cell) keeps key -1 and no deposit
-  const int key = push_tangent_particle(a, win, p, own);
+  bool left = false;
+  const int key = push_tangent_particle(a, win, p, own, left);
+  // (counted per block: one shared counter, an atomic per wave, was three
+  // quarters of the kernel's time, 10 ns for each of its 131072 waves at
+  // 64^3 x 32)
+  const int leaving = __popcll(__ballot(left));
+  if ((threadIdx.x & 63) == 0) wmovers[threadIdx.x >> 6] = leaving;
   deposit_runs(a, win, key, own);
   __syncthreads();
+  if (threadIdx.x == 0) {
+    int all = 0;
+#pragma unroll
+    for (int u = 0; u < kBlock / 64; ++u) all += wmovers[u];
+    a.movers[blockIdx.x] = all;
+  }
   // the window's sums, one global atomic per value that received any
   const size_t N = a.ncells;
   for (int i = threadIdx.x; i < 12 * kTanWindow; i += blockDim.x) {
