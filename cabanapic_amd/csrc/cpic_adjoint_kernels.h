@@ -495,21 +495,19 @@ __device__ __forceinline__ void load_lacc(const AdjointPush<R>& a, int v, double
 // key < 0 for none.
 __device__ __forceinline__ void add_interp_runs(double* linterp, int key, double l[18]) {
   const int lane = threadIdx.x & 63;
-  const int before = __shfl_up(key, 1, 64);
-  int head = (lane == 0 || before != key) ? 1 : 0;
+  int first;
+  bool last;
+  key_run(key, lane, first, last);
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int h = __shfl_up(head, off, 64);
-    const bool add = lane >= off && !head;
+  for (int k0 = 0; k0 < 18; k0 += 6) {
+    double v[6];
 #pragma unroll
-    for (int k = 0; k < 18; ++k) {
-      const double y = __shfl_up(l[k], off, 64);
-      if (add) l[k] += y;
-    }
-    if (lane >= off) head |= h;
+    for (int k = 0; k < 6; ++k) v[k] = l[k0 + k];
+    run_sums(v, lane, first);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) l[k0 + k] = v[k];
   }
-  const int after = __shfl_down(key, 1, 64);
-  if (key >= 0 && (lane == 63 || after != key)) {
+  if (key >= 0 && last) {
     double* li = linterp + (size_t)key * kInterpStride;
 #pragma unroll
     for (int k = 0; k < 18; ++k)

@@ -153,6 +153,54 @@ __device__ __forceinline__ int wave_sum_int(int v) {
 // load cannot be moved past it.
 template <class V> __device__ __forceinline__ void settle(V& v) { asm volatile("" : "+v"(v)); }
 
+// Sums over runs of consecutive lanes of a wave (an inclusive scan that does
+// not cross the lane first, where the lane's run starts).  The values move by
+// DPP, in the vector units: the same scan by ds_bpermute, 216 of them for 12
+// dual numbers or 18 doubles, kept LDS busy for three quarters of the tangent
+// push.  Steps 1, 2, 4 and 8 shift within rows of 16 lanes (the lanes shifted
+// in from outside read 0), the last two add a row's, then a half's, last lane.
+template <int CTRL> __device__ __forceinline__ int dpp_move(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(dpp_move<CTRL>(__float_as_int(v)));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v) {
+  return __hiloint2double(dpp_move<CTRL>(__double2hiint(v)), dpp_move<CTRL>(__double2loint(v)));
+}
+constexpr int kDppRowShr = 0x110, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+
+template <int CTRL, class T, int N>
+__device__ __forceinline__ void run_sum_step(T (&v)[N], bool take) {
+  T from[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) from[k] = dpp_move<CTRL>(v[k]);
+  if (take) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = from[k] + v[k];
+  }
+}
+template <class T, int N>
+__device__ __forceinline__ void run_sums(T (&v)[N], int lane, int first) {
+  run_sum_step<kDppRowShr + 1>(v, lane - 1 >= first);
+  run_sum_step<kDppRowShr + 2>(v, lane - 2 >= first);
+  run_sum_step<kDppRowShr + 4>(v, lane - 4 >= first);
+  run_sum_step<kDppRowShr + 8>(v, lane - 8 >= first);
+  run_sum_step<kDppRowBcast15>(v, (lane & 16) && first < (lane & 48));
+  run_sum_step<kDppRowBcast31>(v, (lane & 32) && first < 32);
+}
+
+// The run of equal keys in consecutive lanes that the calling lane is in
+// (every lane of the wave calls it): its first lane, and whether the lane is
+// its last.
+__device__ __forceinline__ void key_run(int key, int lane, int& first, bool& last) {
+  const int prev = __shfl_up(key, 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || prev != key);
+  const unsigned long long upto = lane == 63 ? heads : heads & ((2ull << lane) - 1);
+  first = 63 - __clzll((long long)upto);
+  last = lane == 63 || ((heads >> (lane + 1)) & 1);
+}
+
 // correction term of a streak (move_p.h:154): real_t product scaled by the
 // double 1/3, rounded back to real_t
 __device__ __forceinline__ float streak_v5(float q, float a, float b, float c) {

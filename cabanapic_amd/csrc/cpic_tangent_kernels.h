@@ -178,25 +178,24 @@ template <class R>
 __device__ __forceinline__ void deposit_runs(const TangentPush<R>& a, const TanWindow<R>& w,
                                              int key, Dual<R> o[12]) {
   const int lane = threadIdx.x & 63;
-  const int before = __shfl_up(key, 1, 64);
-  int head = (lane == 0 || before != key) ? 1 : 0;
+  int first;
+  bool last;
+  key_run(key, lane, first, last);
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int h = __shfl_up(head, off, 64);
-    const bool add = lane >= off && !head;
+  for (int k0 = 0; k0 < 12; k0 += 4) {
+    R v[4];
+    double t[4];
 #pragma unroll
-    for (int k = 0; k < 12; ++k) {
-      const R yv = __shfl_up(o[k].v, off, 64);
-      const double yt = __shfl_up(o[k].t, off, 64);
-      if (add) {
-        o[k].v = yv + o[k].v;
-        o[k].t = yt + o[k].t;
-      }
+    for (int k = 0; k < 4; ++k) {
+      v[k] = o[k0 + k].v;
+      t[k] = o[k0 + k].t;
     }
-    if (lane >= off) head |= h;
+    run_sums(v, lane, first);
+    run_sums(t, lane, first);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k0 + k] = Dual<R>(v[k], t[k]);
   }
-  const int after = __shfl_down(key, 1, 64);
-  if (key >= 0 && (lane == 63 || after != key)) deposit_dual(a, w, key, o);
+  if (key >= 0 && last) deposit_dual(a, w, key, o);
 }
 
 // The push of particle p (nothing for p >= n); returns the voxel of its own
