@@ -22,7 +22,21 @@
 
 namespace cpic {
 
-// A value of type R and its derivative, in FP64.  Operators are hidden
+// 1 / b in FP64 to its last bit or the one beside it: two Newton steps on the
+// hardware's estimate, without the scaling that a full divide does for
+// operands near the ends of the FP64 range, where no FP32 value lies.
+__device__ __forceinline__ double tangent_rcp(float b) {
+  const double d = b;
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.), r, r);
+  return __builtin_fma(__builtin_fma(-d, r, 1.), r, r);
+}
+__device__ __forceinline__ double tangent_rcp(double b) { return 1. / b; }
+
+// A value of type R and its derivative, in FP64.  The values' operations are
+// never contracted; the tangents' products and sums are (one rounding less, and
+// fewer instructions for a kernel that spends 69 % of its time issuing them:
+// 858 -> 816 us for the push of 64^3 x 32).  Operators are hidden
 // friends, so integer and floating constants convert implicitly.
 template <class R> struct Dual {
   R v;
@@ -39,11 +53,11 @@ template <class R> struct Dual {
   }
   friend __device__ __forceinline__ Dual operator-(const Dual& a) { return Dual(-a.v, -a.t); }
   friend __device__ __forceinline__ Dual operator*(const Dual& a, const Dual& b) {
-    return Dual(a.v * b.v, a.t * (double)b.v + (double)a.v * b.t);
+    return Dual(a.v * b.v, __builtin_fma(a.t, (double)b.v, (double)a.v * b.t));
   }
   friend __device__ __forceinline__ Dual operator/(const Dual& a, const Dual& b) {
     const R q = a.v / b.v;
-    return Dual(q, (a.t - (double)q * b.t) / (double)b.v);
+    return Dual(q, __builtin_fma(-(double)q, b.t, a.t) * tangent_rcp(b.v));
   }
   __device__ __forceinline__ Dual& operator+=(const Dual& b) { return *this = *this + b; }
   __device__ __forceinline__ Dual& operator-=(const Dual& b) { return *this = *this - b; }
@@ -57,7 +71,7 @@ template <class R> struct Dual {
 // the narrowed square root of the push and its derivative 1 / (2 sqrt)
 template <class R> __device__ __forceinline__ Dual<R> sqrtf_narrow(const Dual<R>& s) {
   const R r = sqrtf_narrow(s.v);
-  return Dual<R>(r, s.t * 0.5 / (double)r);
+  return Dual<R>(r, s.t * 0.5 * tangent_rcp(r));
 }
 
 // the streak correction term q a b c / 3 and its derivative
@@ -65,7 +79,9 @@ template <class R>
 __device__ __forceinline__ Dual<R> streak_v5(const Dual<R>& q, const Dual<R>& a,
                                              const Dual<R>& b, const Dual<R>& c) {
   const double Q = q.v, A = a.v, B = b.v, C = c.v;
-  const double t = (q.t * A * B * C + Q * a.t * B * C + Q * A * b.t * C + Q * A * B * c.t) * (1. / 3.);
+  const double AB = A * B, dAB = __builtin_fma(a.t, B, A * b.t);
+  const double dABC = __builtin_fma(dAB, C, AB * c.t);
+  const double t = __builtin_fma(q.t, AB * C, Q * dABC) * (1. / 3.);
   return Dual<R>(streak_v5(q.v, a.v, b.v, c.v), t);
 }
 
