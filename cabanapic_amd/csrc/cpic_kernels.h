@@ -297,7 +297,7 @@ __device__ __forceinline__ void for_each_ghost_image(const Grid& g, int x, int y
 template <class R>
 __device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Grid& g, int x,
                                                 int y, int z, int i, R px, R py, R pz,
-                                                double* v = nullptr) {
+                                                R* eb = nullptr) {
   const size_t N = g.ncells;
   const R* ex = fields;
   const R* ey = fields + N;
@@ -317,10 +317,13 @@ __device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Gr
     by[w] = nby;
     bz[w] = nbz;
   });
-  if (v) {
-    const double e0 = e_x, e1 = e_y, e2 = e_z, b0 = nbx, b1 = nby, b2 = nbz;
-    v[0] = e0 * e0 + e1 * e1 + e2 * e2;
-    v[1] = b0 * b0 + b1 * b1 + b2 * b2;
+  if (eb) {  // the voxel's E and new B
+    eb[0] = e_x;
+    eb[1] = e_y;
+    eb[2] = e_z;
+    eb[3] = nbx;
+    eb[4] = nby;
+    eb[5] = nbz;
   }
 }
 
@@ -340,14 +343,8 @@ __global__ void __launch_bounds__(kBlock) k_advance_b(R* __restrict__ fields, Gr
 // reads J from its periodic source (the value the copy gives it), and each
 // interior thread writes its voxel's J into the ghosts it is the source of.
 template <class R>
-__global__ void __launch_bounds__(kBlock)
-k_advance_e(R* __restrict__ fields, Grid g, R px, R py, R pz, R cj) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int mx = g.nx + 1, my = g.ny + 1, mz = g.nz + 1;
-  if (t >= mx * my * mz) return;
-  const int x = 1 + t % mx;
-  const int y = 1 + (t / mx) % my;
-  const int z = 1 + t / (mx * my);
+__device__ __forceinline__ void advance_e_voxel(R* __restrict__ fields, const Grid& g, int x,
+                                                int y, int z, R px, R py, R pz, R cj) {
   const int i = voxel(g, x, y, z);
   const size_t N = g.ncells;
   R* ex = fields;
@@ -373,6 +370,15 @@ k_advance_e(R* __restrict__ fields, Grid g, R px, R py, R pz, R cj) {
       jy[v] = j_y;
       jz[v] = j_z;
     });
+}
+
+template <class R>
+__global__ void __launch_bounds__(kBlock)
+k_advance_e(R* __restrict__ fields, Grid g, R px, R py, R pz, R cj) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int mx = g.nx + 1, my = g.ny + 1, mz = g.nz + 1;
+  if (t >= mx * my * mz) return;
+  advance_e_voxel(fields, g, 1 + t % mx, 1 + (t / mx) % my, 1 + t / (mx * my), px, py, pz, cj);
 }
 
 // ---------------------------------------------------------------------------
@@ -419,7 +425,11 @@ k_advance_b_energy(R* __restrict__ fields, Grid g, R px, R py, R pz,
     const int x = 1 + t % g.nx;
     const int y = 1 + (t / g.nx) % g.ny;
     const int z = 1 + t / (g.nx * g.ny);
-    advance_b_voxel(fields, g, x, y, z, voxel(g, x, y, z), px, py, pz, v);
+    R eb[6];
+    advance_b_voxel(fields, g, x, y, z, voxel(g, x, y, z), px, py, pz, eb);
+    const double e0 = eb[0], e1 = eb[1], e2 = eb[2], b0 = eb[3], b1 = eb[4], b2 = eb[5];
+    v[0] = e0 * e0 + e1 * e1 + e2 * e2;
+    v[1] = b0 * b0 + b1 * b1 + b2 * b2;
   }
   block_sum_store<2>(v, partials + 2 * (size_t)blockIdx.x);
 }

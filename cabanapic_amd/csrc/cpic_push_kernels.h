@@ -1059,29 +1059,16 @@ k_publish_push(const int* __restrict__ grp_rows, int ngroups, const int* err,
   publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
 }
 
-// The field stages between the push and advance_e in one launch (the fused
-// step's; small grids are bound by the number of launches): unload
-// (src/accumulator.cpp:45-122), the J fold (k_fold_j's closed form, from the
-// accumulators directly: a voxel of the high ghost layer is unloaded by the
-// thread whose voxel it folds into) and advance_b with its ghosts, in the
-// order of the separate kernels for every value.  J is written on interior
-// voxels only: k_advance_e, which follows, writes the ghosts.  The last block
-// has no cells and publishes the push's status.
+// The field stages between the push and advance_e at one interior voxel (i, at
+// x, y, z): unload (src/accumulator.cpp:45-122), the J fold (k_fold_j's closed
+// form, from the accumulators directly: a voxel of the high ghost layer is
+// unloaded by the thread whose voxel it folds into) and advance_b with its
+// ghosts, in the order of the separate kernels for every value.  J is written
+// on interior voxels only: advance_e, which follows, writes the ghosts.
 template <class R>
-__global__ void __launch_bounds__(kBlock)
-k_current_advance_b(R* __restrict__ fields, const R* __restrict__ acc, Grid g, R cx, R cy, R cz,
-                    R px, R py, R pz, const int* __restrict__ grp_rows, int ngroups,
-                    const int* err, unsigned* ovf_count, int seq, PushStatus* host) {
-  if (blockIdx.x == gridDim.x - 1) {
-    publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
-    return;
-  }
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= g.nx * g.ny * g.nz) return;
-  const int x = 1 + t % g.nx;
-  const int y = 1 + (t / g.nx) % g.ny;
-  const int z = 1 + t / (g.nx * g.ny);
-  const int i = voxel(g, x, y, z);
+__device__ __forceinline__ void currents_voxel(R* __restrict__ fields, const R* __restrict__ acc,
+                                               const Grid& g, int x, int y, int z, int i, R cx,
+                                               R cy, R cz, R px, R py, R pz) {
   const size_t N = g.ncells;
   const int pos[3] = {x, y, z};
   const int n[3] = {g.nx, g.ny, g.nz};
@@ -1106,6 +1093,26 @@ k_current_advance_b(R* __restrict__ fields, const R* __restrict__ acc, Grid g, R
     fields[(6 + c) * N + i] = J;
   }
   advance_b_voxel(fields, g, x, y, z, i, px, py, pz);
+}
+
+// Those stages in one launch (the fused step's; small grids are bound by the
+// number of launches).  The last block has no cells and publishes the push's
+// status.
+template <class R>
+__global__ void __launch_bounds__(kBlock)
+k_current_advance_b(R* __restrict__ fields, const R* __restrict__ acc, Grid g, R cx, R cy, R cz,
+                    R px, R py, R pz, const int* __restrict__ grp_rows, int ngroups,
+                    const int* err, unsigned* ovf_count, int seq, PushStatus* host) {
+  if (blockIdx.x == gridDim.x - 1) {
+    publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
+    return;
+  }
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= g.nx * g.ny * g.nz) return;
+  const int x = 1 + t % g.nx;
+  const int y = 1 + (t / g.nx) % g.ny;
+  const int z = 1 + t / (g.nx * g.ny);
+  currents_voxel(fields, acc, g, x, y, z, voxel(g, x, y, z), cx, cy, cz, px, py, pz);
 }
 
 // uncenter_particles, src/uncenter_p.h:4-105: for every particle, a
