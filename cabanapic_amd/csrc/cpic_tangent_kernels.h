@@ -331,24 +331,56 @@ __device__ __forceinline__ void wave_key_run(int key, int& first, int& len) {
 // the run sums of the push's own-cell deposits see a cell's particles in
 // consecutive lanes (particles keep drifting out of the order of their
 // upload).  Count: particles per voxel (an invalid voxel counts in bin 0
-// and is flagged by the push), one atomic per run of a voxel in a wave,
-// whose result gives every particle its rank within its voxel.
+// and is flagged by the push), and every particle's rank within its voxel.
+// A block counts in LDS over the voxels that nearly all its particles are in
+// (the push's window and side segments), one atomic per run of a voxel in a
+// wave, and takes a place for all of them with one atomic per voxel: its
+// particles of a voxel then go to consecutive places, too, which the scatter's
+// stores merge.  188 + 509 us for the count and the scatter of 64^3 x 32 with an
+// atomic per run.
 __global__ void __launch_bounds__(kBlock)
-k_tangent_bin_count(const int* __restrict__ cell, int n, int ncells, int* __restrict__ bins,
-                    int* __restrict__ rank) {
+k_tangent_bin_count(const int* __restrict__ cell, int n, int ncells, int sy, int sz,
+                    int* __restrict__ bins, int* __restrict__ rank) {
+  constexpr int kSlots = kTanWindow + 4 * kTanSide;
+  __shared__ int count[kSlots];
+  for (int i = threadIdx.x; i < kSlots; i += blockDim.x) count[i] = 0;
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  const int base = cell[blockIdx.x * blockDim.x] - 1;  // (the block has a first particle)
+  auto side = [&](int s) { return s == 0 ? sy : s == 1 ? -sy : s == 2 ? sz : -sz; };
   int key = -1;
   if (p < n) {
     const int v = cell[p];
     key = (v >= 0 && v < ncells) ? v : 0;
   }
+  int slot = -1;  // the voxel's place in count
+  {
+    const int r = key - base;
+#pragma unroll
+    for (int s = 3; s >= 0; --s) {
+      const unsigned d = (unsigned)(r - side(s));
+      if (d < (unsigned)kTanSide) slot = kTanWindow + kTanSide * s + (int)d;
+    }
+    if ((unsigned)r < (unsigned)kTanWindow) slot = r;
+  }
   int first, len;
   wave_key_run(key, first, len);
   const int lane = threadIdx.x & 63;
-  int base = 0;
-  if (key >= 0 && lane == first) base = atomicAdd(bins + key, len);
-  base = __shfl(base, first, 64);
-  if (key >= 0) rank[p] = base + (lane - first);
+  __syncthreads();
+  int at = 0;
+  if (key >= 0 && lane == first)
+    at = slot >= 0 ? atomicAdd(&count[slot], len) : atomicAdd(bins + key, len);
+  __syncthreads();
+  for (int i = threadIdx.x; i < kSlots; i += blockDim.x) {
+    const int c = count[i];
+    if (c == 0) continue;
+    const int k = i - kTanWindow;
+    const int v = base + (k < 0 ? i : side(k / kTanSide) + k % kTanSide);
+    count[i] = atomicAdd(bins + v, c);
+  }
+  __syncthreads();
+  if (key >= 0 && lane == first && slot >= 0) at += count[slot];
+  at = __shfl(at, first, 64);
+  if (key >= 0) rank[p] = at + (lane - first);
 }
 
 // Scatter: every particle to its voxel's range (start: the exclusive scan
