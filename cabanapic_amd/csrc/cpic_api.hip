@@ -18,6 +18,7 @@
 #include "../../include/cabanapic_amd.h"
 #include "cpic_host_copy.h"
 #include "cpic_push_kernels.h"
+#include "cpic_small_kernels.h"
 #include "cpic_split_kernels.h"
 #include "cpic_tangent_kernels.h"
 #include "cpic_adjoint_kernels.h"
@@ -102,10 +103,11 @@ struct ColumnSet {
   // it writes a record addressed to a cell of the group, cleared by the
   // second, whose waves without a mark have nothing to do
   int* rec_flags = nullptr;
-  // per group, in the same allocation: rows its columns used in the last push
-  // and particles that took the move_p branch
+  // in the same allocation: per group the rows its columns used in the last
+  // push, and the particles that took the move_p branch, in n_movers counts
   int* grp_rows = nullptr;
   int* grp_movers = nullptr;
+  int n_movers = 0;
   // rows that pass 2 took, [MW][nc_pad], for columns of more than
   // kTakenWords words only
   unsigned long long* taken = nullptr;
@@ -306,6 +308,8 @@ ColState<R> col_state(cpic_context* c, int from) {
   return cs;
 }
 
+int column_groups(const cpic_context* c) { return (int)(c->nc_pad / 64); }
+
 // Waves that share a group of 64 cells in pass 1 and in pass 2: 8 where the
 // groups alone do not fill the chip (1024 SIMDs), else 4 and 2.  Pass 1 / pass
 // 2 in us, with 2, 4 and 8 waves: 32^3 cells x 32 (512 groups) 45 29 25 / 23
@@ -318,6 +322,22 @@ struct SplitWaves {
 SplitWaves split_waves(const cpic_context* c) {
   if (cdiv(c->nc, 64) <= 512) return {8, 8};
   return {4, 2};
+}
+
+// Whether the kernels for grids of few cells run: a wave per cell instead of a
+// lane, for up to 4096 cells, whose waves find the chip's 256 CUs mostly idle.
+// A step in us, a wave per cell / a lane, two-stream plasmas in FP32 and FP64:
+//   cells x particles     FP32          FP64
+//   32 x 64               42 / 62       45 / 81
+//   200 x 200             63 / 159      67 / 220
+//   1000 x 16             38 / 46       40 / 53
+//   12^3 x 64             59 / 87       65 / 108
+//   16^3 x 16             52 / 58       57 / 67
+//   16^3 x 200            96 / 170      118 / 212
+//   20^3 x 16             65 / 61       73 / 69
+//   24^3 x 64             114 / 94      149 / 124
+bool small_grid(const cpic_context* c) {
+  return c->nc <= kSmallCells && c->MW <= kSmallWords;
 }
 
 // Whether this push packs the columns: every interval-th one that the caller
@@ -383,7 +403,14 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   // 32-bit byte offsets; columns too deep for that are packed at every push.
   const bool group_fits = (int64_t)c->D * 64 * kSlotLen * (int64_t)sizeof(R) < INT32_MAX;
   const SplitWaves waves = split_waves(c);
-  if (compact || !group_fits)
+  const bool small = small_grid(c);
+  const int cell_blocks = cdiv(c->nc, kSmallWaves);
+  const bool cells = small && !compact && group_fits;
+  c->n_movers = cells ? cell_blocks : column_groups(c);
+  if (cells)
+    c->compensated ? k_push_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p)
+                   : k_push_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p);
+  else if (compact || !group_fits)
     c->compensated ? k_push_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
                    : k_push_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
   else
@@ -407,8 +434,12 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   ar.cdt_dz = cdt_dz;
   ar.qsp = qsp;
   ar.err = c->err;
-  c->compensated ? launch_arrive_split<R, true>(c, ar, waves.arrive)
-                 : launch_arrive_split<R, false>(c, ar, waves.arrive);
+  if (small)
+    c->compensated ? k_arrive_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar)
+                   : k_arrive_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar);
+  else
+    c->compensated ? launch_arrive_split<R, true>(c, ar, waves.arrive)
+                   : launch_arrive_split<R, false>(c, ar, waves.arrive);
   CHECK_LAUNCH();
 
   // the streaks after the 2nd and 3rd crossings, from the record lists
@@ -608,7 +639,9 @@ int alloc_column_set(cpic_context* c, int D, int M1, int M2, ColumnSet& out) {
     if ((t = alloc((void**)&s.ovf_cell, sizeof(int) * s.ovf_cap))) return t;
     if ((t = alloc((void**)&s.dep, sizeof(unsigned long long) * kDepMasks * words))) return t;
     const size_t groups = c->nc_pad / 64;
-    if ((t = alloc((void**)&s.dep_words, sizeof(int) * 4 * groups))) return t;
+    // (movers: k_push_cells counts per block of kSmallWaves cells)
+    const size_t ints = 3 * groups + (size_t)c->nc_pad / kSmallWaves;
+    if ((t = alloc((void**)&s.dep_words, sizeof(int) * ints))) return t;
     if (s.MW > kTakenWords)
       if ((t = alloc((void**)&s.taken, sizeof(unsigned long long) * words))) return t;
     s.rec_flags = s.dep_words + groups;
@@ -619,7 +652,7 @@ int alloc_column_set(cpic_context* c, int D, int M1, int M2, ColumnSet& out) {
       if ((t = fill_zero<unsigned long long>(c, s.mask[b], words))) return t;
     }
     if ((t = fill_zero<unsigned long long>(c, s.dep, kDepMasks * words))) return t;
-    if ((t = fill_zero<int>(c, s.dep_words, 4 * groups))) return t;
+    if ((t = fill_zero<int>(c, s.dep_words, ints))) return t;
     return CPIC_OK;
   };
   if (int t = run()) {
@@ -681,8 +714,6 @@ int check_device_errors(cpic_context* c) {
 // bunching in one cell (a nonlinear two-stream phase reaches 4x the mean
 // count) do not overflow it.  A push that overflows anyway fails with
 // kErrColumnFull.
-
-int column_groups(const cpic_context* c) { return (int)(c->nc_pad / 64); }
 
 // Numbers the push whose status is about to be published (false: no push ran).
 bool next_status(cpic_context* c) {
@@ -1698,10 +1729,10 @@ int cpic_stage_times(cpic_context* c, int64_t* counts, double* ms) {
 int cpic_last_push_movers(cpic_context* c, int64_t* movers) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
-    // counted per block by a tangent push, per group by a column push
+    // counted per block by a tangent push, per group or block by a column push
     const bool columns = c->D > 0 && c->np > 0;
     const int* from = columns ? c->grp_movers : c->block_movers;
-    std::vector<int> per((size_t)(columns ? column_groups(c) : c->n_block_movers));
+    std::vector<int> per((size_t)(columns ? c->n_movers : c->n_block_movers));
     if (!per.empty())
       HIP_TRY(hipMemcpyAsync(per.data(), from, sizeof(int) * per.size(), hipMemcpyDeviceToHost,
                              c->stream));

@@ -572,10 +572,11 @@ template <class R> struct PushPass {
   R qdt_2mc, cdt_dx, cdt_dy, cdt_dz, qsp;
   int accumulate;  // 1: acc += (push semantics), 0: acc = (after a clear)
   int* err;
-  // per group, written by pass 1: rows its columns use, and particles that
-  // took the move_p branch.  One plain store each: an atomic per wave on a
-  // shared counter took longer than the pass itself on small grids (32^3
-  // cells, 2048 waves: 45 us with the atomics)
+  // written by pass 1: per group the rows its columns use, and per group (or
+  // per block of k_push_cells) the particles that took the move_p branch.  One
+  // plain store each: an atomic per wave on a shared counter took longer than
+  // the pass itself on small grids (32^3 cells, 2048 waves: 45 us with the
+  // atomics)
   int* grp_rows;
   int* grp_movers;
 };
