@@ -109,7 +109,7 @@ struct ColumnSet {
   int* grp_movers = nullptr;
   int n_movers = 0;
   // rows that pass 2 took, [MW][nc_pad], for columns of more than
-  // kTakenWords words only
+  // kTakenWords words only (kSmallWords is more)
   unsigned long long* taken = nullptr;
 };
 
@@ -336,9 +336,7 @@ SplitWaves split_waves(const cpic_context* c) {
 //   16^3 x 200            96 / 170      118 / 212
 //   20^3 x 16             65 / 61       73 / 69
 //   24^3 x 64             114 / 94      149 / 124
-bool small_grid(const cpic_context* c) {
-  return c->nc <= kSmallCells && c->MW <= kSmallWords;
-}
+bool small_grid(const cpic_context* c) { return c->nc <= kSmallCells; }
 
 // Whether this push packs the columns: every interval-th one that the caller
 // names, by default every kCompactInterval-th of a grid that fills the chip.

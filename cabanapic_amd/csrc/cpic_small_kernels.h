@@ -15,7 +15,7 @@
 namespace cpic {
 
 constexpr int kSmallWaves = 4;      // cells per block: a 128-byte line of FP32 slots
-constexpr int kSmallWords = 64;     // mask words per cell that the small kernels take
+constexpr int kSmallWords = 16;     // mask words whose taken rows k_arrive_cells notes in LDS
 constexpr int kSmallCells = 4096;   // cells of a grid that uses them
 
 // Contributions of up to 64 rows, padded against bank conflicts, and the sums
@@ -28,6 +28,7 @@ template <class R, bool K> struct CellSums {
   __device__ __forceinline__ void add(Rows& rows, int lane, int n, const R o[12]) {
 #pragma unroll
     for (int k = 0; k < 12; ++k) rows[lane][k] = o[k];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     if (lane < 12) {
       for (int r = 0; r < n; ++r) {
@@ -42,6 +43,7 @@ template <class R, bool K> struct CellSums {
         }
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
   __device__ __forceinline__ void store(R* acc, size_t N, int v, int lane, bool onto) const {
@@ -159,7 +161,17 @@ __global__ void __launch_bounds__(64 * kSmallWaves) k_arrive_cells(ArrivePass<R>
   const int src = sel6(lane < 6 ? lane : 0, nb[3], nb[4], nb[5], nb[0], nb[1], nb[2]);
   const int written = lane < 6 ? a.dep_words[src >> 6] : 0;
   const int nw = min(wave_max_int(written), MW);
-  for (int w = lane; w < MW; w += 64) taken[wave][w] = 0;
+  // rows handed out: in LDS, and for the words of columns that are deeper (a
+  // grid of few particles has rows for all of them) in global memory, where
+  // the lines of other cells' words are shared, so past the vector cache
+  unsigned long long* const deep = a.taken + ci;
+  for (int w = lane; w < MW; w += 64) {
+    if (w < kSmallWords)
+      taken[wave][w] = 0;
+    else
+      __hip_atomic_store(&deep[(size_t)w * MP], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (MW > kSmallWords) __threadfence();
   const unsigned long long* const occ = a.cs.mask_out + ci;
   int hw = 0;  // the first word with free rows that are still to be had, and those
   unsigned long long freeb = ~occ[0] & low_bits(D);
@@ -244,7 +256,11 @@ __global__ void __launch_bounds__(64 * kSmallWaves) k_arrive_cells(ArrivePass<R>
       if (f == 6) {
         if (row >= 0) {
           store_particle(a.cs, ci, row, pos[0], pos[1], pos[2], pa.w, pb.x, pb.y, pb.z, pb.w);
-          atomicOr(&taken[wave][row >> 6], 1ull << (row & 63));
+          const unsigned long long bit = 1ull << (row & 63);
+          if (row < 64 * kSmallWords)
+            atomicOr(&taken[wave][row >> 6], bit);
+          else
+            atomicOr(&deep[(size_t)(row >> 6) * MP], bit);
         } else {
           atomicOr(a.err, kErrColumnFull);
         }
@@ -257,8 +273,12 @@ __global__ void __launch_bounds__(64 * kSmallWaves) k_arrive_cells(ArrivePass<R>
   }
   // the rows taken become occupied, those of the cell's own departures free
   const int own_words = min(a.dep_words[ci >> 6], MW);
+  if (MW > kSmallWords) __threadfence();
   for (int w = lane; w < MW; w += 64) {
-    const unsigned long long add = taken[wave][w];
+    const unsigned long long add =
+        w < kSmallWords ? taken[wave][w]
+                        : __hip_atomic_load(&deep[(size_t)w * MP], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long own = w < own_words ? a.dep[dep_index(6, w, MW, MP, ci)] : 0ull;
     if (add | own) {
       unsigned long long* m = a.cs.mask_out + (size_t)w * MP + ci;

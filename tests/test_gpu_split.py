@@ -1,8 +1,7 @@
 """The passes whose rows and arrivals several waves share, and those with a wave
 per cell, at the sizes where they can go wrong: groups of 64 cells that are
 partly filled, columns around a mask word and past what one chunk of words
-holds, columns too deep for LDS (which also take small grids to the shared
-passes), both wave counts (up to 512 groups of cells, and more), 4096 cells and
+holds, columns too deep for LDS, both wave counts (up to 512 groups of cells, and more), 4096 cells and
 4097, more arrivals than lanes, and steps without some of the energies.  Particles equal the oracle's bit for bit;
 accumulators agree within the bound of a reordered sum (as in
 test_gpu_parity.py)."""
@@ -21,7 +20,8 @@ CASES = [
     (5, 13, 1, 2, 0, 3), (3, 2, 1, 300, 0, 3), (4, 1, 1, 9, 4200, 3),
     (32, 32, 32, 2, 0, 2), (33, 32, 32, 2, 0, 2),
     (16, 16, 16, 9, 0, 2), (241, 17, 1, 9, 0, 2), (3, 2, 1, 900, 0, 3),
-    (63, 1, 1, 3, 4200, 3), (65, 1, 1, 65, 4200, 2), (3, 2, 1, 300, 4200, 3),
+    (63, 1, 1, 3, 4200, 3), (3, 1, 1, 1500, 0, 3), (241, 17, 1, 1, 0, 3),
+    (241, 17, 1, 65, 0, 2), (241, 17, 1, 300, 0, 2),
 ]
 
 
