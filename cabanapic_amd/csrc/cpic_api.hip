@@ -844,11 +844,12 @@ int snapshot_begin(cpic_context* c, int slot) {
   if (!c->copy_stream)
     HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
   char* d = (char*)sn.dev;
-  const long nthreads = std::max<long>(std::max<long>(c->nc, c->nx), 3);
+  const int groups = column_groups(c);
+  const dim3 grid(groups, std::clamp(1024 / groups, 1, 16));
   const bool have = c->np > 0 && c->D > 0;
   int s = with_real(c, [&](auto r) -> int {
     using R = decltype(r);
-    k_snapshot<R><<<cdiv(nthreads, kBlock), kBlock, 0, c->stream>>>(
+    k_snapshot<R><<<grid, kBlock, 0, c->stream>>>(
         have ? (const R*)c->cols[c->cur] : nullptr, have ? c->cnt[c->cur] : nullptr,
         have ? c->mask[c->cur] : nullptr, c->cg, c->D, (int)c->nc_pad, have ? c->np : 0,
         (const R*)c->fields, c->grid.sy, c->grid.sz, c->red_out, (R*)(d + L.x),

@@ -86,3 +86,19 @@ def test_snapshot_keeps_its_layout_across_an_upload():
             assert_bitwise(snap["ux"], s.p["ux"], f"ux, slot {slot}")
             assert_bitwise(snap["cell"], s.cell, f"cell, slot {slot}")
         assert sim.device_errors() == 0
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 1, 1, 200), (64, 1, 1, 63), (65, 1, 1, 65),
+                                   (300, 1, 1, 5), (33, 32, 32, 3)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_snapshot_shapes(shape, dtype):
+    """Rows of a group spread over blocks: one cell, columns around a mask
+    word and past one, a line of more cells than a block has threads, more
+    groups of cells than share a row's blocks."""
+    st, _ = states.random_state(*shape, dtype, seed=shape[0] + shape[3])
+    sp = dict(states.step_consts(dtype), energy_interval=1)
+    with sim_from_state(st) as a:
+        a.step_async(sp, 2)
+        a.snapshot_begin(1)
+        _check(a, a.snapshot_wait(1), st)
