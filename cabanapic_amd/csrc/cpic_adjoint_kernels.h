@@ -25,7 +25,7 @@
 // output voxel sums what the forward stage's outputs read from it.
 #pragma once
 
-#include "cpic_push_kernels.h"
+#include "cpic_tangent_kernels.h"
 
 namespace cpic {
 
@@ -221,19 +221,22 @@ __device__ __forceinline__ void quadrants_bwd(R q, R dA, R mB, R mC, const doubl
   const R s1b = s1a + t;
   const R cp = R(1) + mC;
   const R cm = R(1) - mC;
-  lv5 += l[0] - l[1] - l[2] + l[3];
-  // s0b = s0a cm, s1c = s1b cm, s2 = s0a cp, s3 = s1b cp
-  double ls0a = l[0] * (double)cm + l[2] * (double)cp;
-  double ls1b = l[1] * (double)cm + l[3] * (double)cp;
-  lmC += -(l[0] * (double)s0a + l[1] * (double)s1b) + (l[2] * (double)s0a + l[3] * (double)s1b);
-  // s1b = s1a + t, s0a = t - s1a
-  double ls1a = ls1b - ls0a;
-  double lt = ls1b + ls0a;
-  // s1a = t mB
-  lt += ls1a * (double)mB;
-  lmB += ls1a * (double)t;
-  // t = q dA (q carries no derivative)
-  ldA += lt * (double)q;
+  {
+#pragma clang fp contract(fast)
+    lv5 += l[0] - l[1] - l[2] + l[3];
+    // s0b = s0a cm, s1c = s1b cm, s2 = s0a cp, s3 = s1b cp
+    double ls0a = l[0] * (double)cm + l[2] * (double)cp;
+    double ls1b = l[1] * (double)cm + l[3] * (double)cp;
+    lmC += -(l[0] * (double)s0a + l[1] * (double)s1b) + (l[2] * (double)s0a + l[3] * (double)s1b);
+    // s1b = s1a + t, s0a = t - s1a
+    double ls1a = ls1b - ls0a;
+    double lt = ls1b + ls0a;
+    // s1a = t mB
+    lt += ls1a * (double)mB;
+    lmB += ls1a * (double)t;
+    // t = q dA (q carries no derivative)
+    ldA += lt * (double)q;
+  }
 }
 
 // streak_values transposed: l[12] adjoint of the 12 contributions.
@@ -246,26 +249,37 @@ __device__ __forceinline__ void streak_values_bwd(R q, R dx, R dy, R dz, R mx, R
   quadrants_bwd(q, dz, mx, my, l + 8, ld[2], lm[0], lm[1], lv5);
 }
 
-// the streak correction term q a b c / 3 (move_p.h:154), transposed as the
-// tangent differentiates it (in FP64 from the primal operands)
+// The deposit's correction term q a b c / 3, transposed as the tangent
+// differentiates it: a streak's (move_p.h:154) in FP64 from the primal
+// operands, that of a particle that stays in its cell (whole) from the primal
+// products as they were rounded.
 template <class R>
-__device__ __forceinline__ void streak_v5_bwd(R q, R a, R b, R c, double lv5, double& la,
-                                              double& lb, double& lc) {
+__device__ __forceinline__ void streak_v5_bwd(R q, R a, R b, R c, bool whole, double lv5,
+                                              double& la, double& lb, double& lc) {
   const double Q = q, A = a, B = b, C = c;
-  const double s = lv5 * (1. / 3.);
-  la += s * Q * B * C;
-  lb += s * Q * A * C;
-  lc += s * Q * A * B;
+  const R one_third = 1. / 3.;
+  const R t1 = q * a, t2 = t1 * b;
+  const double third = whole ? (double)one_third : 1. / 3.;
+  const double qa = whole ? (double)t1 : Q * A;
+  {
+#pragma clang fp contract(fast)
+    const double s = lv5 * third, sc = s * C;
+    la += sc * B * Q;
+    lb += sc * qa;
+    lc += s * (whole ? (double)t2 : qa * B);
+  }
 }
 
 // One streak (streak() of cpic_push_kernels.h) transposed.  pos, rem: the
 // streak's inputs; lpos, lrem: on entry the adjoints of its outputs (pos and
 // rem after the streak), on exit those of its inputs.  lacc: adjoint of the
-// accumulators of the streak's cell.  Returns the face crossed (as streak).
+// accumulators of the streak's cell.  whole: the particle stays in its cell
+// and rem is the whole displacement (the push's own deposit is that of a
+// streak that no face ends).
 template <class R>
-__device__ __forceinline__ int streak_bwd(const R pos[3], const R rem[3], R q,
-                                          const double lacc[12], double lpos[3],
-                                          double lrem[3]) {
+__device__ __forceinline__ void streak_bwd(const R pos[3], const R rem[3], R q, bool whole,
+                                           const double lacc[12], double lpos[3],
+                                           double lrem[3]) {
   R dir[3], len3[3], dsp0[3], dsp[3], mid[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -276,9 +290,11 @@ __device__ __forceinline__ int streak_bwd(const R pos[3], const R rem[3], R q,
   }
   R len = 2;
   int axis = 3;
-  if (len3[0] < len) len = len3[0], axis = 0;
-  if (len3[1] < len) len = len3[1], axis = 1;
-  if (len3[2] < len) len = len3[2], axis = 2;
+  if (!whole) {
+    if (len3[0] < len) len = len3[0], axis = 0;
+    if (len3[1] < len) len = len3[1], axis = 1;
+    if (len3[2] < len) len = len3[2], axis = 2;
+  }
   const R lenh = len * R(0.5);
   R mid1[3];
 #pragma unroll
@@ -286,44 +302,40 @@ __device__ __forceinline__ int streak_bwd(const R pos[3], const R rem[3], R q,
     dsp[k] = dsp0[k] * lenh;
     mid1[k] = mid[k] + dsp[k];
   }
-  const R v5 = streak_v5(q, dsp[0], dsp[1], dsp[2]);
-  (void)v5;
-  // the snap of the crossed coordinate: its output carries no derivative
-  double lp[3] = {lpos[0], lpos[1], lpos[2]};
-  if (axis < 3) lp[axis] = 0;
-  double ldsp[3], lmid1[3] = {0, 0, 0}, lv5 = 0;
+  {
+#pragma clang fp contract(fast)
+    // the snap of the crossed coordinate: its output carries no derivative
+    double lp[3] = {lpos[0], lpos[1], lpos[2]};
+    R crossed = 1;  // rem on the crossed axis
 #pragma unroll
-  for (int k = 0; k < 3; ++k) ldsp[k] = -lrem[k] + 2.0 * lp[k];  // rem -= dsp; pos += 2 dsp
-  streak_values_bwd(q, dsp[0], dsp[1], dsp[2], mid1[0], mid1[1], mid1[2], lacc, ldsp, lmid1, lv5);
-  streak_v5_bwd(q, dsp[0], dsp[1], dsp[2], lv5, ldsp[0], ldsp[1], ldsp[2]);
-  // mid1 = mid + dsp
-  double lmid[3];
+    for (int k = 0; k < 3; ++k)
+      if (axis == k) lp[k] = 0, crossed = dsp0[k];
+    double ldsp[3], lmid1[3] = {0, 0, 0}, lv5 = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    lmid[k] = lmid1[k];
-    ldsp[k] += lmid1[k];
-  }
-  // dsp = dsp0 lenh
-  double llenh = 0, ldsp0[3];
+    for (int k = 0; k < 3; ++k) ldsp[k] = -lrem[k] + 2.0 * lp[k];  // rem -= dsp; pos += 2 dsp
+    streak_values_bwd(q, dsp[0], dsp[1], dsp[2], mid1[0], mid1[1], mid1[2], lacc, ldsp, lmid1,
+                      lv5);
+    streak_v5_bwd(q, dsp[0], dsp[1], dsp[2], whole, lv5, ldsp[0], ldsp[1], ldsp[2]);
+    // mid1 = mid + dsp; dsp = dsp0 lenh
+    double llenh = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    ldsp0[k] = ldsp[k] * (double)lenh;
-    llenh += ldsp[k] * (double)dsp0[k];
-  }
-  if (axis < 3) {
+    for (int k = 0; k < 3; ++k) {
+      ldsp[k] += lmid1[k];
+      llenh += ldsp[k] * (double)dsp0[k];
+    }
     // lenh = 0.5 len, len = (dir - mid) / dsp0 on the crossed axis
-    const double llen = 0.5 * llenh;
-    const double b = dsp0[axis];
-    lmid[axis] -= llen / b;
-    ldsp0[axis] -= llen * (double)len / b;
-  }
+    const double lb = 0.5 * llenh * tangent_rcp(crossed);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    lpos[k] = lp[k] + lmid[k];
-    lrem[k] += ldsp0[k];
+    for (int k = 0; k < 3; ++k) {
+      double lm = lmid1[k], ld0 = ldsp[k] * (double)lenh;
+      if (axis == k) {
+        lm -= lb;
+        ld0 -= lb * (double)len;
+      }
+      lpos[k] = lp[k] + lm;
+      lrem[k] += ld0;
+    }
   }
-  if (axis == 3) return -1;
-  return axis + ((dir[axis] > 0) ? 3 : 0);
 }
 
 // displacement() transposed: ld adjoint of (ddx, ddy, ddz); adds to lu.
@@ -337,16 +349,20 @@ __device__ __forceinline__ void displacement_bwd(R ux, R uy, R uz, R cdt_dx, R c
   const R a[3] = {ux * cdt_dx, uy * cdt_dy, uz * cdt_dz};
   const R c[3] = {cdt_dx, cdt_dy, cdt_dz};
   const R u[3] = {ux, uy, uz};
-  double lv0 = 0;
+  {
+#pragma clang fp contract(fast)
+    double lv0 = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    lv0 += ld[k] * (double)a[k];
-    lu[k] += ld[k] * (double)v0 * (double)c[k];
+    for (int k = 0; k < 3; ++k) {
+      lv0 += ld[k] * (double)a[k];
+      lu[k] += ld[k] * ((double)v0 * (double)c[k]);
+    }
+    // v0 = 1 / r, r = sqrt(s), s = 1 + |u|^2: ls 2 u
+    const double ri = tangent_rcp(r);
+    const double ls2 = -lv0 * (double)v0 * ri * ri;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) lu[k] += ls2 * (double)u[k];
   }
-  const double lr = -lv0 * (double)v0 / (double)r;
-  const double ls = lr * 0.5 / (double)r;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) lu[k] += ls * 2.0 * (double)u[k];
 }
 
 // boris() transposed.  Inputs: the interpolator (e0..b1) and the particle
@@ -387,83 +403,86 @@ __device__ __forceinline__ void boris_bwd(const V4& e0, const V4& e1, const V4& 
   const R w0 = ux + v3 * X0, w1 = uy + v3 * X1, w2 = uz + v3 * X2;
   const R Y0 = w1 * cbz - w2 * cby, Y1 = w2 * cbx - w0 * cbz, Y2 = w0 * cby - w1 * cbx;
   // backward: u3 = u2 + ha, u2 = u1 + v4 Y
-  const double lha[3] = {lu[0], lu[1], lu[2]};
-  double lu1[3] = {lu[0], lu[1], lu[2]};
-  double lv4 = lu[0] * (double)Y0 + lu[1] * (double)Y1 + lu[2] * (double)Y2;
-  const double lY0 = lu[0] * (double)v4, lY1 = lu[1] * (double)v4, lY2 = lu[2] * (double)v4;
-  double lw0 = 0, lw1 = 0, lw2 = 0, lcbx = 0, lcby = 0, lcbz = 0;
-  // Y0 = w1 cbz - w2 cby
-  lw1 += lY0 * (double)cbz; lcbz += lY0 * (double)w1; lw2 -= lY0 * (double)cby; lcby -= lY0 * (double)w2;
-  // Y1 = w2 cbx - w0 cbz
-  lw2 += lY1 * (double)cbx; lcbx += lY1 * (double)w2; lw0 -= lY1 * (double)cbz; lcbz -= lY1 * (double)w0;
-  // Y2 = w0 cby - w1 cbx
-  lw0 += lY2 * (double)cby; lcby += lY2 * (double)w0; lw1 -= lY2 * (double)cbx; lcbx -= lY2 * (double)w1;
-  // w = u1 + v3 X
-  lu1[0] += lw0; lu1[1] += lw1; lu1[2] += lw2;
-  double lv3 = lw0 * (double)X0 + lw1 * (double)X1 + lw2 * (double)X2;
-  const double lX0 = lw0 * (double)v3, lX1 = lw1 * (double)v3, lX2 = lw2 * (double)v3;
-  // X0 = uy cbz - uz cby
-  lu1[1] += lX0 * (double)cbz; lcbz += lX0 * (double)uy; lu1[2] -= lX0 * (double)cby; lcby -= lX0 * (double)uz;
-  // X1 = uz cbx - ux cbz
-  lu1[2] += lX1 * (double)cbx; lcbx += lX1 * (double)uz; lu1[0] -= lX1 * (double)cbz; lcbz -= lX1 * (double)ux;
-  // X2 = ux cby - uy cbx
-  lu1[0] += lX2 * (double)cby; lcby += lX2 * (double)ux; lu1[1] -= lX2 * (double)cbx; lcbx -= lX2 * (double)uy;
-  // v4 = 2 v4a, v4a = v3 / den, den = 1 + v1 v3sq
-  const double lv4a = 2.0 * lv4;
-  lv3 += lv4a / (double)den;
-  const double lden = -lv4a * (double)v4a / (double)den;
-  double lv1 = lden * (double)v3sq;
-  lv3 += lden * (double)v1 * 2.0 * (double)v3;
-  // v3 = v0 poly, poly = 1 + v2 inner, inner = 1/3 + v2 2/15
-  double lv0 = lv3 * (double)poly;
-  const double lpoly = lv3 * (double)v0;
-  double lv2 = lpoly * (double)inner;
-  lv2 += lpoly * (double)v2 * (double)two_fifteenths;
-  // v2 = v0sq v1
-  lv1 += lv2 * (double)v0sq;
-  lv0 += lv2 * (double)v1 * 2.0 * (double)v0;
-  // v1 = |cb|^2
-  lcbx += lv1 * 2.0 * (double)cbx;
-  lcby += lv1 * 2.0 * (double)cby;
-  lcbz += lv1 * 2.0 * (double)cbz;
-  // v0 = qdt_2mc / r, r = sqrt(s), s = 1 + |u1|^2
-  const double lr = -lv0 * (double)v0 / (double)r;
-  const double ls = lr * 0.5 / (double)r;
-  lu1[0] += ls * 2.0 * (double)ux;
-  lu1[1] += ls * 2.0 * (double)uy;
-  lu1[2] += ls * 2.0 * (double)uz;
-  // u1 = u0 + ha
-  lu[0] = lu1[0];
-  lu[1] = lu1[1];
-  lu[2] = lu1[2];
-  const double lhx = lha[0] + lu1[0], lhy = lha[1] + lu1[1], lhz = lha[2] + lu1[2];
-  // cbx = b0.x + dx b0.y, cby = b0.z + dy b0.w, cbz = b1.x + dz b1.y
-  lf[12] += lcbx; ld[0] += lcbx * (double)b0.y; lf[13] += lcbx * (double)dx;
-  lf[14] += lcby; ld[1] += lcby * (double)b0.w; lf[15] += lcby * (double)dy;
-  lf[16] += lcbz; ld[2] += lcbz * (double)b1.y; lf[17] += lcbz * (double)dz;
-  // hax = q ((e0.x + dy e0.y) + dz (e0.z + dy e0.w))
   {
-    const double li = lhx * (double)qdt_2mc;
-    lf[0] += li; ld[1] += li * (double)e0.y; lf[1] += li * (double)dy;
-    ld[2] += li * (double)zx;
-    const double lz = li * (double)dz;
-    lf[2] += lz; ld[1] += lz * (double)e0.w; lf[3] += lz * (double)dy;
-  }
-  // hay = q ((e1.x + dz e1.y) + dx (e1.z + dz e1.w))
-  {
-    const double li = lhy * (double)qdt_2mc;
-    lf[4] += li; ld[2] += li * (double)e1.y; lf[5] += li * (double)dz;
-    ld[0] += li * (double)zy;
-    const double lz = li * (double)dx;
-    lf[6] += lz; ld[2] += lz * (double)e1.w; lf[7] += lz * (double)dz;
-  }
-  // haz = q ((e2.x + dx e2.y) + dy (e2.z + dx e2.w))
-  {
-    const double li = lhz * (double)qdt_2mc;
-    lf[8] += li; ld[0] += li * (double)e2.y; lf[9] += li * (double)dx;
-    ld[1] += li * (double)zz;
-    const double lz = li * (double)dy;
-    lf[10] += lz; ld[0] += lz * (double)e2.w; lf[11] += lz * (double)dx;
+#pragma clang fp contract(fast)
+    const double lha[3] = {lu[0], lu[1], lu[2]};
+    double lu1[3] = {lu[0], lu[1], lu[2]};
+    double lv4 = lu[0] * (double)Y0 + lu[1] * (double)Y1 + lu[2] * (double)Y2;
+    const double lY0 = lu[0] * (double)v4, lY1 = lu[1] * (double)v4, lY2 = lu[2] * (double)v4;
+    double lw0 = 0, lw1 = 0, lw2 = 0, lcbx = 0, lcby = 0, lcbz = 0;
+    // Y0 = w1 cbz - w2 cby
+    lw1 += lY0 * (double)cbz; lcbz += lY0 * (double)w1; lw2 -= lY0 * (double)cby; lcby -= lY0 * (double)w2;
+    // Y1 = w2 cbx - w0 cbz
+    lw2 += lY1 * (double)cbx; lcbx += lY1 * (double)w2; lw0 -= lY1 * (double)cbz; lcbz -= lY1 * (double)w0;
+    // Y2 = w0 cby - w1 cbx
+    lw0 += lY2 * (double)cby; lcby += lY2 * (double)w0; lw1 -= lY2 * (double)cbx; lcbx -= lY2 * (double)w1;
+    // w = u1 + v3 X
+    lu1[0] += lw0; lu1[1] += lw1; lu1[2] += lw2;
+    double lv3 = lw0 * (double)X0 + lw1 * (double)X1 + lw2 * (double)X2;
+    const double lX0 = lw0 * (double)v3, lX1 = lw1 * (double)v3, lX2 = lw2 * (double)v3;
+    // X0 = uy cbz - uz cby
+    lu1[1] += lX0 * (double)cbz; lcbz += lX0 * (double)uy; lu1[2] -= lX0 * (double)cby; lcby -= lX0 * (double)uz;
+    // X1 = uz cbx - ux cbz
+    lu1[2] += lX1 * (double)cbx; lcbx += lX1 * (double)uz; lu1[0] -= lX1 * (double)cbz; lcbz -= lX1 * (double)ux;
+    // X2 = ux cby - uy cbx
+    lu1[0] += lX2 * (double)cby; lcby += lX2 * (double)ux; lu1[1] -= lX2 * (double)cbx; lcbx -= lX2 * (double)uy;
+    // v4 = 2 v4a, v4a = v3 / den, den = 1 + v1 v3sq
+    const double lv4a = 2.0 * lv4 * tangent_rcp(den);  // over den
+    lv3 += lv4a;
+    const double lden = -lv4a * (double)v4a;
+    double lv1 = lden * (double)v3sq;
+    lv3 += lden * (double)v1 * 2.0 * (double)v3;
+    // v3 = v0 poly, poly = 1 + v2 inner, inner = 1/3 + v2 2/15
+    double lv0 = lv3 * (double)poly;
+    const double lpoly = lv3 * (double)v0;
+    double lv2 = lpoly * (double)inner;
+    lv2 += lpoly * (double)v2 * (double)two_fifteenths;
+    // v2 = v0sq v1
+    lv1 += lv2 * (double)v0sq;
+    lv0 += lv2 * (double)v1 * 2.0 * (double)v0;
+    // v1 = |cb|^2
+    lcbx += lv1 * 2.0 * (double)cbx;
+    lcby += lv1 * 2.0 * (double)cby;
+    lcbz += lv1 * 2.0 * (double)cbz;
+    // v0 = qdt_2mc / r, r = sqrt(s), s = 1 + |u1|^2
+    const double ri = tangent_rcp(r);
+    const double ls2 = -lv0 * (double)v0 * ri * ri;
+    lu1[0] += ls2 * (double)ux;
+    lu1[1] += ls2 * (double)uy;
+    lu1[2] += ls2 * (double)uz;
+    // u1 = u0 + ha
+    lu[0] = lu1[0];
+    lu[1] = lu1[1];
+    lu[2] = lu1[2];
+    const double lhx = lha[0] + lu1[0], lhy = lha[1] + lu1[1], lhz = lha[2] + lu1[2];
+    // cbx = b0.x + dx b0.y, cby = b0.z + dy b0.w, cbz = b1.x + dz b1.y
+    lf[12] += lcbx; ld[0] += lcbx * (double)b0.y; lf[13] += lcbx * (double)dx;
+    lf[14] += lcby; ld[1] += lcby * (double)b0.w; lf[15] += lcby * (double)dy;
+    lf[16] += lcbz; ld[2] += lcbz * (double)b1.y; lf[17] += lcbz * (double)dz;
+    // hax = q ((e0.x + dy e0.y) + dz (e0.z + dy e0.w))
+    {
+      const double li = lhx * (double)qdt_2mc;
+      lf[0] += li; ld[1] += li * (double)e0.y; lf[1] += li * (double)dy;
+      ld[2] += li * (double)zx;
+      const double lz = li * (double)dz;
+      lf[2] += lz; ld[1] += lz * (double)e0.w; lf[3] += lz * (double)dy;
+    }
+    // hay = q ((e1.x + dz e1.y) + dx (e1.z + dz e1.w))
+    {
+      const double li = lhy * (double)qdt_2mc;
+      lf[4] += li; ld[2] += li * (double)e1.y; lf[5] += li * (double)dz;
+      ld[0] += li * (double)zy;
+      const double lz = li * (double)dx;
+      lf[6] += lz; ld[2] += lz * (double)e1.w; lf[7] += lz * (double)dz;
+    }
+    // haz = q ((e2.x + dx e2.y) + dy (e2.z + dx e2.w))
+    {
+      const double li = lhz * (double)qdt_2mc;
+      lf[8] += li; ld[0] += li * (double)e2.y; lf[9] += li * (double)dx;
+      ld[1] += li * (double)zz;
+      const double lz = li * (double)dy;
+      lf[10] += lz; ld[0] += lz * (double)e2.w; lf[11] += lz * (double)dx;
+    }
   }
 }
 
@@ -472,7 +491,7 @@ template <class R> struct AdjointPush {
   const int* cell;     // [n] interior cell of each snapshot slot
   long n;
   const R* interp;     // the step's interpolators (cell-major, kInterpStride)
-  const double* lacc;  // adjoint of the accumulators, slot-major [12][Ng]
+  const double* lacc;  // [Ng][12]: adjoint of the accumulators
   const double* lout;  // [n][kAdjRec]: adjoint of the step's output particles, by tag
   double* lin;         // [n][kAdjRec]: adjoint of its input particles, by tag
   double* linterp;     // [Ng][kInterpStride]: adjoint of the interpolators (added to)
@@ -484,34 +503,49 @@ template <class R> struct AdjointPush {
 
 template <class R>
 __device__ __forceinline__ void load_lacc(const AdjointPush<R>& a, int v, double l[12]) {
-  const size_t N = a.ncells;
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  const D2* p = reinterpret_cast<const D2*>(a.lacc + (size_t)v * 12);
 #pragma unroll
-  for (int k = 0; k < 12; ++k) l[k] = a.lacc[k * N + v];
+  for (int k = 0; k < 6; ++k) {
+    const D2 t = p[k];
+    l[2 * k] = t.x;
+    l[2 * k + 1] = t.y;
+  }
 }
 
-// Sums l[18] over each run of consecutive lanes of the wave with the same
-// key (a segmented inclusive scan; the last lane of a run then adds the
-// run's total to linterp of voxel key).  Every lane of the wave calls it;
-// key < 0 for none.
-__device__ __forceinline__ void add_interp_runs(double* linterp, int key, double l[18]) {
+// Interpolator adjoints of a wave's lanes on their way to linterp.
+struct InterpRows {
+  double l[18][65];  // (odd stride: 18 lanes read one row of it)
+  int key[64];
+};
+
+// Adds l[18] of each lane of the wave to linterp of voxel key (< 0 for none),
+// summed over runs of lanes with the same key first.  54 lanes walk a third of
+// the rows each for one of the 18 values: some 60 instructions, where segmented
+// scans of 18 values by DPP were 500 of the push's 2160.  Every lane of the
+// wave calls it.
+__device__ __forceinline__ void add_interp_runs(double* linterp, int key, const double l[18],
+                                                InterpRows& rows) {
   const int lane = threadIdx.x & 63;
-  int first;
-  bool last;
-  key_run(key, lane, first, last);
+  const int prev = __shfl_up(key, 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || prev != key);
+  const unsigned long long ends = heads >> 1 | 1ull << 63;
 #pragma unroll
-  for (int k0 = 0; k0 < 18; k0 += 6) {
-    double v[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) v[k] = l[k0 + k];
-    run_sums(v, lane, first);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) l[k0 + k] = v[k];
-  }
-  if (key >= 0 && last) {
-    double* li = linterp + (size_t)key * kInterpStride;
-#pragma unroll
-    for (int k = 0; k < 18; ++k)
-      if (l[k] != 0.0) unsafeAtomicAdd(li + k, l[k]);
+  for (int k = 0; k < 18; ++k) rows.l[k][lane] = l[k];
+  rows.key[lane] = key;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (lane >= 54) return;
+  constexpr int kRows = 22;
+  const int k = lane % 18, r0 = lane / 18 * kRows, r1 = min(r0 + kRows, 64);
+  double s = 0;
+  for (int r = r0; r < r1; ++r) {
+    s += rows.l[k][r];
+    if ((ends >> r & 1) || r == r1 - 1) {
+      const int v = rows.key[r];
+      if (v >= 0 && s != 0.0) unsafeAtomicAdd(linterp + (size_t)v * kInterpStride + k, s);
+      s = 0;
+    }
   }
 }
 
@@ -521,8 +555,16 @@ __device__ __forceinline__ void add_interp_runs(double* linterp, int key, double
 // reverse).  Writes the input-particle adjoint by tag; the interpolator
 // adjoints of the cell's particles are summed over the wave's runs of lanes
 // in one cell and added atomically.
+//
+// Bound by the vector units' FP64 instructions.  A particle that stays in its
+// cell takes the streaks' own code, since nearly every wave holds some that
+// leave it; the adjoints' products and sums are contracted (the primal values
+// are not); the interpolator sums go through LDS; a cell's accumulator adjoints
+// lie together.  32^3 x 32 in FP32: 71 us, 88 before those four.  A fourth wave
+// per SIMD (128 registers) spills: 113 us.
 template <class R>
 __global__ void __launch_bounds__(kBlock) k_push_adjoint(AdjointPush<R> a) {
+  __shared__ InterpRows interp_rows[kBlock / 64];
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   double lf[18];
 #pragma unroll
@@ -537,7 +579,6 @@ __global__ void __launch_bounds__(kBlock) k_push_adjoint(AdjointPush<R> a) {
     const V4* sl = reinterpret_cast<const V4*>(a.slots + (size_t)p * kSlotLen);
     const V4 pa = sl[0], pb = sl[1];
     const R one = 1.;
-    const R one_third = 1. / 3.;
     const R dx = pa.x, dy = pa.y, dz = pa.z;
     const R ux0 = pa.w, uy0 = pb.x, uz0 = pb.y, w = pb.z;
     const long t = TagBits<R>::get(pb.w);
@@ -557,59 +598,48 @@ __global__ void __launch_bounds__(kBlock) k_push_adjoint(AdjointPush<R> a) {
       const double* lo = a.lout + (size_t)t * kAdjRec;
       double lpos[3] = {lo[0], lo[1], lo[2]};
       double lu[3] = {lo[3], lo[4], lo[5]};
-      double ld[3] = {0, 0, 0}, ldd[3] = {0, 0, 0};
-      double lacc[12];
-      if (nx <= one && ny <= one && nz <= one && -nx <= one && -ny <= one && -nz <= one) {
-        // in-cell: pos' = (d + dd) + dd, deposit with v5 = q ddx ddy ddz / 3
-        load_lacc(a, v, lacc);
-        const R t1 = q * dd[0], t2 = t1 * dd[1];
-        double lm[3] = {0, 0, 0}, lv5 = 0;
-        streak_values_bwd(q, dd[0], dd[1], dd[2], mx, my, mz, lacc, ldd, lm, lv5);
-        const double lt3 = lv5 * (double)one_third;
-        const double lt2 = lt3 * (double)dd[2];
-        ldd[2] += lt3 * (double)t2;
-        const double lt1 = lt2 * (double)dd[1];
-        ldd[1] += lt2 * (double)t1;
-        ldd[0] += lt1 * (double)q;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          // m = d + dd, n = m + dd
-          const double lmk = lm[k] + lpos[k];
-          ldd[k] += lpos[k] + lmk;
-          ld[k] += lmk;
-        }
-      } else {
-        // the streaks: recount them forward, then transpose the last first
-        int K = 0;
-        {
-          R pos[3] = {dx, dy, dz}, rem[3] = {dd[0], dd[1], dd[2]};
-          R dsp[3], mid[3], v5;
-          for (; K < kMaxStreaks; ++K) {
-            if (streak_geometry(pos, rem, q, dsp, mid, v5) < 0) break;
-          }
-          ++K;
-          if (K > kMaxStreaks) {
+      const bool whole =
+          nx <= one && ny <= one && nz <= one && -nx <= one && -ny <= one && -nz <= one;
+      // the streaks: recount them forward, keeping where the second starts (few
+      // particles have more), then transpose the last first
+      int K = 1;
+      R pos1[3] = {0, 0, 0}, rem1[3] = {0, 0, 0};
+      int cell1 = ci;
+      if (!whole) {
+        R pos[3] = {dx, dy, dz}, rem[3] = {dd[0], dd[1], dd[2]};
+        R dsp[3], mid[3], v5;
+        for (;; ++K) {
+          const int face = streak_geometry(pos, rem, q, dsp, mid, v5);
+          if (face < 0) break;
+          if (K == kMaxStreaks) {
             atomicOr(a.err, kErrStreakLimit);
-            K = kMaxStreaks;
+            break;
           }
-        }
-        double lrem[3] = {0, 0, 0};  // the remainder after the last streak is no output
-        for (int s = K - 1; s >= 0; --s) {
-          // inputs and cell of streak s
-          R pos[3] = {dx, dy, dz}, rem[3] = {dd[0], dd[1], dd[2]};
-          int cs = ci;
-          R dsp[3], mid[3], v5;
-          for (int k = 0; k < s; ++k)
-            cs = face_neighbor(a.g, cs, streak_geometry(pos, rem, q, dsp, mid, v5));
-          load_lacc(a, interior_to_voxel(a.g, cs), lacc);
-          streak_bwd(pos, rem, q, lacc, lpos, lrem);
-        }
+          if (K == 1) {
+            cell1 = face_neighbor(a.g, ci, face);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          ld[k] = lpos[k];
-          ldd[k] = lrem[k];
+            for (int k = 0; k < 3; ++k) pos1[k] = pos[k], rem1[k] = rem[k];
+          }
         }
       }
+      double ldd[3] = {0, 0, 0};  // the remainder after the last streak is no output
+      for (int s = K - 1; s >= 0; --s) {
+        // inputs and cell of streak s
+        R pos[3] = {dx, dy, dz}, rem[3] = {dd[0], dd[1], dd[2]};
+        int cs = ci;
+        if (s > 0) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k) pos[k] = pos1[k], rem[k] = rem1[k];
+          cs = cell1;
+          R dsp[3], mid[3], v5;
+          for (int k = 1; k < s; ++k)
+            cs = face_neighbor(a.g, cs, streak_geometry(pos, rem, q, dsp, mid, v5));
+        }
+        double lacc[12];
+        load_lacc(a, interior_to_voxel(a.g, cs), lacc);
+        streak_bwd(pos, rem, q, whole, lacc, lpos, ldd);
+      }
+      double ld[3] = {lpos[0], lpos[1], lpos[2]};
       displacement_bwd(ux, uy, uz, a.cdt_dx, a.cdt_dy, a.cdt_dz, ldd, lu);
       boris_bwd(e0, e1, e2, b0, b1, a.qdt_2mc, dx, dy, dz, ux0, uy0, uz0, lu, ld, lf);
       double* li = a.lin + (size_t)t * kAdjRec;
@@ -621,7 +651,7 @@ __global__ void __launch_bounds__(kBlock) k_push_adjoint(AdjointPush<R> a) {
       reinterpret_cast<D4*>(li)[1] = r1;
     }
   }
-  add_interp_runs(a.linterp, key, lf);
+  add_interp_runs(a.linterp, key, lf, interp_rows[threadIdx.x >> 6]);
 }
 
 // ---------------------------------------------------------------------------
@@ -709,19 +739,19 @@ k_unload_bwd(const double* __restrict__ lf, double* __restrict__ lacc, Grid g, d
   const double* jy = lf + 7 * N;
   const double* jz = lf + 8 * N;
   const int sy = g.sy, sz = g.sz;
-  double* A = lacc;
-  A[0 * N + v] = cx * jx[v];
-  A[1 * N + v] = cx * jx[v + sy];
-  A[2 * N + v] = cx * jx[v + sz];
-  A[3 * N + v] = cx * jx[v + sy + sz];
-  A[4 * N + v] = cy * jy[v];
-  A[5 * N + v] = cy * jy[v + sz];
-  A[6 * N + v] = cy * jy[v + 1];
-  A[7 * N + v] = cy * jy[v + 1 + sz];
-  A[8 * N + v] = cz * jz[v];
-  A[9 * N + v] = cz * jz[v + 1];
-  A[10 * N + v] = cz * jz[v + sy];
-  A[11 * N + v] = cz * jz[v + 1 + sy];
+  double* A = lacc + (size_t)v * 12;
+  A[0] = cx * jx[v];
+  A[1] = cx * jx[v + sy];
+  A[2] = cx * jx[v + sz];
+  A[3] = cx * jx[v + sy + sz];
+  A[4] = cy * jy[v];
+  A[5] = cy * jy[v + sz];
+  A[6] = cy * jy[v + 1];
+  A[7] = cy * jy[v + 1 + sz];
+  A[8] = cz * jz[v];
+  A[9] = cz * jz[v + 1];
+  A[10] = cz * jz[v + sy];
+  A[11] = cz * jz[v + 1 + sy];
 }
 
 // the J adjoint after the transposed unload: J is overwritten by every step,

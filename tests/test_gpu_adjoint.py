@@ -265,3 +265,29 @@ def test_gradient_is_the_same_with_buffers_in_place():
     for o in first[1:]:
         for a, b in zip(first[0][1:], o[1:]):
             assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32], ids=_name)
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 1, 1, 300), (2, 1, 3, 64), (3, 2, 1, 23),
+                                   (16, 1, 1, 5), (65, 1, 1, 130)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_one_step_of_particles_to_a_wave(shape, dtype):
+    """Cells of one particle, of a part of a wave, of several waves; many
+    particles crossing two and three faces.  The bound of
+    test_one_step_matches_oracle_adjoint: only the order of the sums differs."""
+    st, _ = states.random_state(*shape, dtype, seed=sum(shape), umax=3.0)
+    st.p["w"][:] = (st.p["w"] * 0.05).astype(dtype)
+    k = states.step_consts(dtype)
+    rng = np.random.default_rng(9)
+    seed_f = rng.uniform(-1, 1, (9, st.ng))
+    seed_p = rng.uniform(-1, 1, (6, st.np))
+    with _sim(st) as sim, Adjoint(sim) as adj:
+        adj.forward(dict(k, energy_interval=0), 1, 1, history=False)
+        gf, gp = adj.backward(seed_f, seed_p)
+        assert sim.device_errors() == 0
+    lf = seed_f.copy()
+    lp = st.step_adjoint(states.consts_vector(k), lf, seed_p)
+    ok_f, ef = _close(gf, lf, 1e-12)
+    ok_p, ep = _close(gp, lp, 1e-12)
+    print(f"{_name(dtype)} {shape}: fields {ef:.2e}, particles {ep:.2e}")
+    assert ok_f and ok_p, (ef, ep)
