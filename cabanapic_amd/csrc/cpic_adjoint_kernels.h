@@ -104,52 +104,65 @@ k_scan_add(int* __restrict__ out, int n, const int* __restrict__ sums) {
     if (base + k < n) out[base + k] += add;
 }
 
-// The context's columns into a snapshot: lane per cell, each occupied row
-// (in row order) copied as its whole slot to slots[first[ci] + k]; cell[]
-// receives the interior cell index of every snapshot slot.  Rows are taken
-// kSnapRows at a time: the batch's loads are all issued before its stores,
-// and the batch's slots land next to each other, so each lane completes
-// its output lines in a few consecutive stores.
-constexpr int kSnapRows = 4;
-static_assert(64 % kSnapRows == 0, "a mask word holds whole batches of rows");
+// The position of set bit n (from 0) of m, which has more.
+__device__ __forceinline__ int nth_set_bit(unsigned long long m, int n) {
+  int at = 0;
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    const int c = __popcll(m & ((1ull << w) - 1));
+    if (n >= c) n -= c, at += w, m >>= w;
+  }
+  return at;
+}
+
+// The context's columns into a snapshot: each occupied row (in row order) of
+// cell ci copied as its whole slot to slots[first[ci] + k]; cell[] receives
+// the interior cell index of every snapshot slot.  A block per group of 64
+// cells, whose slots lie together in the snapshot, and a thread per slot, which
+// looks up the cell and the row that it comes from: the stores are whole lines
+// and the loads, 32-byte sectors, are the block's own lines.  A lane per column
+// (512 waves at 32^3 x 32) took 45 us, a wave per 4 rows of a group 31 (lines
+// completed by several waves); so 19.
+constexpr int kSnapBlock = 512;
 
 template <class R>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kSnapBlock)
 k_snapshot_columns(const R* __restrict__ cols, const int* __restrict__ cnt,
                    const unsigned long long* __restrict__ mask, int nc, int nc_pad, int D,
                    const int* __restrict__ first, R* __restrict__ slots, int* __restrict__ cell) {
   typedef typename Vec4T<R>::type V4;
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ci >= nc) return;
-  const int len = min(cnt[ci], D);
-  long o = first[ci];
-  const long end = first[ci + 1];
-  unsigned long long m = 0;
-  for (int j0 = 0; j0 < len && o < end; j0 += kSnapRows) {
-    // j0 is a multiple of kSnapRows, so a new mask word starts only at u = 0
-    if ((j0 & 63) == 0) m = mask[(size_t)(j0 >> 6) * nc_pad + ci];
-    V4 a[kSnapRows], b[kSnapRows];
-    bool occ[kSnapRows];
+  __shared__ int start[65], rows[64];
+  __shared__ unsigned long long occ[64];  // the first mask words
+  const int c0 = blockIdx.x * 64;
+  if (threadIdx.x <= 64) start[threadIdx.x] = first[min(c0 + (int)threadIdx.x, nc)];
+  if (threadIdx.x < 64) {
+    const int ci = c0 + threadIdx.x;  // < nc_pad
+    const int len = ci < nc ? min(cnt[ci], D) : 0;
+    rows[threadIdx.x] = len;
+    occ[threadIdx.x] = mask[ci] & low_bits(len);
+  }
+  __syncthreads();
+  for (int o = start[0] + threadIdx.x; o < start[64]; o += kSnapBlock) {
+    int c = 0;  // the last cell that starts at o or before it
 #pragma unroll
-    for (int u = 0; u < kSnapRows; ++u) {
-      const int j = j0 + u;
-      occ[u] = j < len && ((m >> (j & 63)) & 1ull);
-      if (occ[u]) {
-        const V4* s = reinterpret_cast<const V4*>(cols + col_slot(ci, j, D) * kSlotLen);
-        a[u] = s[0];
-        b[u] = s[1];
-      }
+    for (int w = 32; w > 0; w >>= 1)
+      if (start[c + w] <= o) c += w;
+    int k = o - start[c], word = 0;
+    unsigned long long m = occ[c];
+    for (int n = __popcll(m); k >= n; n = __popcll(m)) {
+      k -= n;
+      const int left = rows[c] - 64 * ++word;
+      if (left <= 0) break;
+      m = mask[(size_t)word * nc_pad + c0 + c] & low_bits(left);
     }
-#pragma unroll
-    for (int u = 0; u < kSnapRows; ++u) {
-      if (occ[u] && o < end) {
-        V4* d = reinterpret_cast<V4*>(slots + (size_t)o * kSlotLen);
-        d[0] = a[u];
-        d[1] = b[u];
-        cell[o] = ci;
-        ++o;
-      }
-    }
+    if (64 * word >= rows[c]) continue;
+    const int j = 64 * word + nth_set_bit(m, k);
+    const V4* s = reinterpret_cast<const V4*>(cols + col_slot(c0 + c, j, D) * kSlotLen);
+    const V4 a = s[0], b = s[1];
+    V4* d = reinterpret_cast<V4*>(slots + (size_t)o * kSlotLen);
+    d[0] = a;
+    d[1] = b;
+    cell[o] = c0 + c;
   }
 }
 

@@ -291,3 +291,26 @@ def test_one_step_of_particles_to_a_wave(shape, dtype):
     ok_p, ep = _close(gp, lp, 1e-12)
     print(f"{_name(dtype)} {shape}: fields {ef:.2e}, particles {ep:.2e}")
     assert ok_f and ok_p, (ef, ep)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (3, 1, 1, 150), (64, 1, 1, 64), (65, 1, 1, 40)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_gradient_from_snapshots_of_columns_with_holes(shape):
+    """Snapshots taken of columns with free rows in and between their mask
+    words: the gradient over a segment of steps equals that with a checkpoint
+    at every step, which starts each step from packed columns.  Both order the
+    same FP64 terms differently: the bound of the five-step test."""
+    st, _ = states.random_state(*shape, F64, seed=shape[0] + 7, umax=0.8)
+    k = dict(states.step_consts(F64), energy_interval=0)
+    rng = np.random.default_rng(4)
+    sf = rng.uniform(-1, 1, (9, st.ng))
+    sp = rng.uniform(-1, 1, (6, st.np))
+    out = []
+    for every in (1, 6):
+        with _sim(st) as sim, Adjoint(sim) as adj:
+            adj.forward(k, 6, every, history=False)
+            out.append(adj.backward(sf, sp))
+            assert sim.device_errors() == 0
+    for a, b in zip(*out):
+        ok, err = _close(a, b, 1e-9)
+        assert ok, err
