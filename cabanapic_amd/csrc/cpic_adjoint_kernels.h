@@ -676,7 +676,9 @@ __device__ __forceinline__ bool in_box(int x, int y, int z, int lo, int hx, int 
 
 // load_interpolator_array transposed: adds to the E and B adjoints what
 // the interior cells' interpolator adjoints (cell-major, kInterpStride) read
-// from every voxel.  One thread per voxel of [1, n+1]^3.
+// from every voxel, and clears the J adjoint, since every step overwrites J and
+// nothing before the step depends on it (the ghosts' is clear already).  One
+// thread per voxel of [1, n+1]^3.
 __global__ void __launch_bounds__(kBlock)
 k_load_interpolator_bwd(double* __restrict__ lf, const double* __restrict__ li, Grid g) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -735,14 +737,18 @@ k_load_interpolator_bwd(double* __restrict__ lf, const double* __restrict__ li, 
   if (cell_ok(0, 0, 0)) s += 0.5 * (L(j, 16) - L(j, 17));
   if (cell_ok(0, 0, 1)) s += 0.5 * (L(j - g.sz, 16) + L(j - g.sz, 17));
   lf[5 * N + j] += s;
+  lf[6 * N + j] = lf[7 * N + j] = lf[8 * N + j] = 0;
 }
 
-// unload_accumulator_array transposed: the accumulator adjoint of every
-// interior cell from the J adjoint over [1, n+1]^3, which the forward
-// stage overwrites (so its adjoint is cleared afterwards, k_clear_j_bwd).
+// What the transposed push takes, for every interior cell: the accumulator
+// adjoint (unload_accumulator_array transposed) from the J adjoint over
+// [1, n+1]^3, the step's interpolators from its fields, and the interpolator
+// adjoints cleared.
+template <class R>
 __global__ void __launch_bounds__(kBlock)
 k_unload_bwd(const double* __restrict__ lf, double* __restrict__ lacc, Grid g, double cx,
-             double cy, double cz) {
+             double cy, double cz, const R* __restrict__ fields, R* __restrict__ interp,
+             double* __restrict__ linterp) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= g.nx * g.ny * g.nz) return;
   const int x = 1 + t % g.nx, y = 1 + (t / g.nx) % g.ny, z = 1 + t / (g.nx * g.ny);
@@ -765,17 +771,13 @@ k_unload_bwd(const double* __restrict__ lf, double* __restrict__ lacc, Grid g, d
   A[9] = cz * jz[v + 1];
   A[10] = cz * jz[v + sy];
   A[11] = cz * jz[v + 1 + sy];
+  typedef typename Vec4T<R>::type V4;
+  V4* dst = reinterpret_cast<V4*>(interp + (size_t)v * kInterpStride);
+  interpolator_at(fields, N, sy, sz, v, dst[0], dst[1], dst[2], dst[3], dst[4]);
+  double* li = linterp + (size_t)v * kInterpStride;
+#pragma unroll
+  for (int k = 0; k < kInterpStride; ++k) li[k] = 0;
 }
-
-// the J adjoint after the transposed unload: J is overwritten by every step,
-// so nothing before the step depends on it
-__global__ void __launch_bounds__(kBlock) k_clear_j_bwd(double* __restrict__ lf, Grid g) {
-  const size_t N = g.ncells;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 3 * N;
-       i += (size_t)gridDim.x * blockDim.x)
-    lf[6 * N + i] = 0;
-}
-
 // advance_b transposed (B_a -= p (E_b(i+s) - E_b(i)) on interior i): B's
 // adjoint is unchanged; E's adjoint at voxel j of [1, n+1]^3 gains what the
 // interior cells that read E(j) contribute.
@@ -858,45 +860,34 @@ k_advance_e_bwd(double* __restrict__ lf, Grid g, double px, double py, double pz
 // The periodic ghost copy transposed, for three components from comp0:
 // every interior voxel gains the adjoints of the ghosts that are its images
 // (each coordinate c also appears as ghost 0 when c = n and as ghost n+1
-// when c = 1), then (k_zero_ghosts_bwd) the ghost adjoints are cleared.
+// when c = 1) and clears them.
 __global__ void __launch_bounds__(kBlock)
 k_copy_ghosts_bwd(double* __restrict__ lf, int comp0, Grid g) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= g.nx * g.ny * g.nz) return;
   const int x = 1 + t % g.nx, y = 1 + (t / g.nx) % g.ny, z = 1 + t / (g.nx * g.ny);
-  int ax[3], ay[3], az[3], nax = 0, nay = 0, naz = 0;
-  ax[nax++] = x;
-  if (x == g.nx) ax[nax++] = 0;
-  if (x == 1) ax[nax++] = g.nx + 1;
-  ay[nay++] = y;
-  if (y == g.ny) ay[nay++] = 0;
-  if (y == 1) ay[nay++] = g.ny + 1;
-  az[naz++] = z;
-  if (z == g.nz) az[naz++] = 0;
-  if (z == 1) az[naz++] = g.nz + 1;
-  if (nax * nay * naz == 1) return;
+  // the coordinate itself, then its images (bit 1: ghost 0, bit 2: ghost n+1)
+  auto images = [](int c, int n) { return 1 | (c == n ? 2 : 0) | (c == 1 ? 4 : 0); };
+  auto at = [](int u, int c, int n) { return u == 0 ? c : u == 1 ? 0 : n + 1; };
+  const int bx = images(x, g.nx), by = images(y, g.ny), bz = images(z, g.nz);
+  if ((bx | by | bz) == 1) return;
   const int j = voxel(g, x, y, z);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    double* a = lf + (size_t)(comp0 + c) * g.ncells;
-    double s = 0;
-    for (int i = 0; i < nax; ++i)
-      for (int k = 0; k < nay; ++k)
-        for (int m = 0; m < naz; ++m)
-          if (i || k || m) s += a[voxel(g, ax[i], ay[k], az[m])];
-    a[j] += s;
-  }
-}
-
-__global__ void __launch_bounds__(kBlock)
-k_zero_ghosts_bwd(double* __restrict__ lf, int comp0, Grid g) {
-  const int X = g.nx + 2, Y = g.ny + 2, Z = g.nz + 2;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= X * Y * Z) return;
-  const int x = t % X, y = (t / X) % Y, z = t / (X * Y);
-  if (x >= 1 && x <= g.nx && y >= 1 && y <= g.ny && z >= 1 && z <= g.nz) return;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) lf[(size_t)(comp0 + c) * g.ncells + t] = 0;
+  const size_t N = g.ncells;
+  double* a = lf + (size_t)comp0 * N;
+  double s0 = 0, s1 = 0, s2 = 0;
+  for (int i = 0; i < 3; ++i)
+    for (int k = 0; k < 3; ++k)
+      for (int m = 0; m < 3; ++m) {
+        if (!((i | k | m) && (bx >> i & 1) && (by >> k & 1) && (bz >> m & 1))) continue;
+        double* p = a + voxel(g, at(i, x, g.nx), at(k, y, g.ny), at(m, z, g.nz));
+        s0 += p[0];
+        s1 += p[N];
+        s2 += p[2 * N];
+        p[0] = p[N] = p[2 * N] = 0;
+      }
+  a[j] += s0;
+  a[N + j] += s1;
+  a[2 * N + j] += s2;
 }
 
 // k_fold_j transposed: every interior face value the fold wrote is a sum of
