@@ -1041,8 +1041,17 @@ __device__ __forceinline__ void publish_push(const int* __restrict__ grp_rows, i
                                              const int* err, unsigned* ovf_count, int seq,
                                              PushStatus* host) {
   __shared__ int part[kBlock / 64];
+  // 16 loads of a thread in flight: one after the other they took 85 us of the
+  // launch for the 32768 groups of 128^3 cells, and 12 for 4096
+  constexpr int kAtOnce = 16;
   int m = 0;
-  for (int i = threadIdx.x; i < ngroups; i += kBlock) m = max(m, grp_rows[i]);
+  for (int i0 = threadIdx.x; i0 < ngroups; i0 += kAtOnce * kBlock) {
+    int r[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) r[u] = grp_rows[min(i0 + u * kBlock, ngroups - 1)];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) m = max(m, r[u]);
+  }
   m = wave_max_int(m);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
   __syncthreads();
@@ -1097,18 +1106,18 @@ __device__ __forceinline__ void currents_voxel(R* __restrict__ fields, const R* 
 }
 
 // Those stages in one launch (the fused step's; small grids are bound by the
-// number of launches).  The last block has no cells and publishes the push's
+// number of launches).  The first block has no cells and publishes the push's
 // status.
 template <class R>
 __global__ void __launch_bounds__(kBlock)
 k_current_advance_b(R* __restrict__ fields, const R* __restrict__ acc, Grid g, R cx, R cy, R cz,
                     R px, R py, R pz, const int* __restrict__ grp_rows, int ngroups,
                     const int* err, unsigned* ovf_count, int seq, PushStatus* host) {
-  if (blockIdx.x == gridDim.x - 1) {
+  if (blockIdx.x == 0) {
     publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
     return;
   }
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
   if (t >= g.nx * g.ny * g.nz) return;
   const int x = 1 + t % g.nx;
   const int y = 1 + (t / g.nx) % g.ny;
