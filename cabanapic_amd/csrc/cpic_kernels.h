@@ -290,14 +290,11 @@ __device__ __forceinline__ void for_each_ghost_image(const Grid& g, int x, int y
         if (c < nzs && b < nys && a < nxs && (a | b | c)) f(voxel(g, xs[a], ys[b], zs[c]));
 }
 
-// EM_Field_Solver::advance_b (src/fields.h:668-719), interior cells, then
-// the periodic ghost copy of B (serial_update_ghosts_B, src/fields.h:11-100):
-// each thread also writes its voxel's new B into the ghosts it is the source
-// of (no thread reads B ghosts here).
+// EM_Field_Solver::advance_b (src/fields.h:668-719) at interior voxel i; eb: its
+// E and new B.
 template <class R>
-__device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Grid& g, int x,
-                                                int y, int z, int i, R px, R py, R pz,
-                                                R* eb = nullptr) {
+__device__ __forceinline__ void advance_b_at(R* fields, const Grid& g, int i, R px, R py, R pz,
+                                             R eb[6]) {
   const size_t N = g.ncells;
   const R* ex = fields;
   const R* ey = fields + N;
@@ -306,24 +303,34 @@ __device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Gr
   R* by = fields + 4 * N;
   R* bz = fields + 5 * N;
   const R e_x = ex[i], e_y = ey[i], e_z = ez[i];
-  const R nbx = bx[i] - (py * (ez[i + g.sy] - e_z) - pz * (ey[i + g.sz] - e_y));
-  const R nby = by[i] - (pz * (ex[i + g.sz] - e_x) - px * (ez[i + 1] - e_z));
-  const R nbz = bz[i] - (px * (ey[i + 1] - e_y) - py * (ex[i + g.sy] - e_x));
-  bx[i] = nbx;
-  by[i] = nby;
-  bz[i] = nbz;
+  eb[0] = e_x;
+  eb[1] = e_y;
+  eb[2] = e_z;
+  eb[3] = bx[i] - (py * (ez[i + g.sy] - e_z) - pz * (ey[i + g.sz] - e_y));
+  eb[4] = by[i] - (pz * (ex[i + g.sz] - e_x) - px * (ez[i + 1] - e_z));
+  eb[5] = bz[i] - (px * (ey[i + 1] - e_y) - py * (ex[i + g.sy] - e_x));
+  bx[i] = eb[3];
+  by[i] = eb[4];
+  bz[i] = eb[5];
+}
+
+// The same, then the periodic ghost copy of B (serial_update_ghosts_B,
+// src/fields.h:11-100): each thread also writes its voxel's new B into the
+// ghosts it is the source of (no thread reads B ghosts here).
+template <class R>
+__device__ __forceinline__ void advance_b_voxel(R* __restrict__ fields, const Grid& g, int x,
+                                                int y, int z, int i, R px, R py, R pz,
+                                                R* eb = nullptr) {
+  const size_t N = g.ncells;
+  R now[6];
+  advance_b_at(fields, g, i, px, py, pz, now);
   for_each_ghost_image(g, x, y, z, [&](int w) {
-    bx[w] = nbx;
-    by[w] = nby;
-    bz[w] = nbz;
+#pragma unroll
+    for (int c = 3; c < 6; ++c) fields[c * N + w] = now[c];
   });
   if (eb) {  // the voxel's E and new B
-    eb[0] = e_x;
-    eb[1] = e_y;
-    eb[2] = e_z;
-    eb[3] = nbx;
-    eb[4] = nby;
-    eb[5] = nbz;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) eb[c] = now[c];
   }
 }
 

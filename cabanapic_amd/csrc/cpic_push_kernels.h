@@ -813,22 +813,24 @@ __device__ __forceinline__ int sel6(int d, int a0, int a1, int a2, int a3, int a
 // Passes 2-4: the next streak of every particle that entered the lane's cell.
 // Each lane walks its own arrivals (all directions, in direction then record
 // order) in one loop, so a wave iterates max over lanes of the lane totals.
+// failed: the error flags, looked at when the loads issued with theirs are back.
+// Returns whether the lane wrote a record (or overflow entry).
+//
+// On grids that leave the chip idle the pass is a chain of load latencies, so
+// loads wait for others only where their address does: counts, occupancy and
+// error flags go together, then the records and the accumulators that the
+// lane's sums will be added to.
 template <class R, bool K>
-__global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
-  if (__builtin_amdgcn_readfirstlane(*a.err)) return;  // this push already failed
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
-  if (a.flag_skip) {
-    // no record of the previous pass is addressed to this wave's cells
-    const int gi = __builtin_amdgcn_readfirstlane(ci >> 6);
-    if (__builtin_amdgcn_readfirstlane(a.flag_skip[gi]) == 0) return;
-    if ((threadIdx.x & 63) == 0) a.flag_skip[gi] = 0;
-  }
+__device__ __forceinline__ bool finish_cell(const FinishPass<R>& a, int ci, int failed) {
   const bool valid = ci < a.g.nc;
   const size_t NC = a.g.nc;
   int s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0;
   int c0 = 0, c1 = 0, c2 = 0, c3 = 0, c4 = 0, c5 = 0;
-  int v = 0;
+  int v = 0, len = 0;
+  unsigned long long w0 = 0;
   if (valid) {
+    len = a.cs.cnt_out[ci];
+    w0 = a.cs.mask_out[ci];
     // the source of a record of direction d sits across the opposite face
     int nb[6];
     face_neighbors6(a.g, ci, nb, v);
@@ -845,17 +847,17 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
     c4 = a.in.cnt[4 * NC + s4];
     c5 = a.in.cnt[5 * NC + s5];
   }
+  if (__builtin_amdgcn_readfirstlane(failed)) return false;
   const int total = c0 + c1 + c2 + c3 + c4 + c5;
   const int tmax = wave_max_int(total);
   int kd[6] = {0, 0, 0, 0, 0, 0};
+  bool crossed = false;
   if (tmax > 0) {
     RowCursor<R> rows;
-    {
-      const int l = valid ? min(a.cs.cnt_out[ci], a.cs.D) : 0;
-      unsigned long long w0 = valid ? a.cs.mask_out[ci] : 0ull;
-      asm volatile("" : "+v"(w0));  // wait for the word here, before the loop
-      rows.start(l, w0);
-    }
+    settle(w0);  // wait for the word here, before the loop
+    rows.start(min(len, a.cs.D), w0);
+    const size_t N = a.ncells;
+    R was[12];
     LaneAcc<R, K> acc;
     acc.zero();
     typedef typename Vec4T<R>::type V4;
@@ -892,6 +894,7 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
         else
           atomicOr(a.err, kErrColumnFull);
       } else {
+        crossed = true;
         int kk = a.last ? a.out.M : kd[d2];  // last pass: straight to overflow
         put_record(a.out, a.ovf, a.g, ci, d2, kk, pos, rem, ux, uy, uz, w, tag, a.err);
         if (!a.last) kd[d2] = kk;
@@ -902,6 +905,10 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
       V4 r0[kRecBatch], r1[kRecBatch], r2[kRecBatch];
 #pragma unroll
       for (int u = 0; u < kRecBatch; ++u) request(i0 + u, r0[u], r1[u], r2[u]);
+      if (i0 == 0 && total > 0) {
+#pragma unroll
+        for (int kq = 0; kq < 12; ++kq) was[kq] = a.acc[kq * N + v];
+      }
 #pragma unroll
       for (int u = 0; u < kRecBatch; ++u) {
         settle(r0[u]);
@@ -916,9 +923,8 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
       rows.finish(a.cs, ci);
       a.cs.cnt_out[ci] = rows.len;
       if (total > 0) {
-        const size_t N = a.ncells;
 #pragma unroll
-        for (int kq = 0; kq < 12; ++kq) a.acc[kq * N + v] += acc.total(kq);
+        for (int kq = 0; kq < 12; ++kq) a.acc[kq * N + v] = was[kq] + acc.total(kq);
       }
     }
   }
@@ -927,6 +933,21 @@ __global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
     for (int dd = 0; dd < 6; ++dd)
       a.out.cnt[(size_t)dd * NC + ci] = (unsigned char)min(kd[dd], a.out.M);
   }
+  return crossed;
+}
+
+template <class R, bool K>
+__global__ void __launch_bounds__(kBlock) k_finish_pass(FinishPass<R> a) {
+  const int failed = *a.err;  // this push already
+  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a.flag_skip) {
+    // no record of the previous pass is addressed to this wave's cells
+    const int gi = __builtin_amdgcn_readfirstlane(ci >> 6);
+    const int marked = a.flag_skip[gi];
+    if (__builtin_amdgcn_readfirstlane(failed) || __builtin_amdgcn_readfirstlane(marked) == 0) return;
+    if ((threadIdx.x & 63) == 0) a.flag_skip[gi] = 0;
+  }
+  finish_cell<R, K>(a, ci, failed);
 }
 
 template <class R> struct ArrivePass {
@@ -976,12 +997,12 @@ template <class R> struct SpillPass {
   int* err;
 };
 
+// Entries first, first + stride, ... of the total in the list.
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_spill_pass(SpillPass<R> a) {
-  if (__builtin_amdgcn_readfirstlane(*a.err)) return;  // this push already failed
-  const unsigned total = min(*a.ovf.count, (unsigned)a.ovf.cap);
+__device__ __forceinline__ void spill_records(const SpillPass<R>& a, unsigned total, unsigned first,
+                                              unsigned stride) {
   typedef typename Vec4T<R>::type V4;
-  for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
+  for (unsigned i = first; i < total; i += stride) {
     const V4* src = reinterpret_cast<const V4*>(a.ovf.rec + (size_t)i * RecordLen<R>::value);
     const V4 r0 = src[0], r1 = src[1], r2 = src[2];
     R pos[3] = {r0.x, r0.y, r0.z};
@@ -1024,6 +1045,13 @@ __global__ void __launch_bounds__(kBlock) k_spill_pass(SpillPass<R> a) {
       atomicOr(a.err, kErrColumnFull);
     }
   }
+}
+
+template <class R>
+__global__ void __launch_bounds__(kBlock) k_spill_pass(SpillPass<R> a) {
+  if (__builtin_amdgcn_readfirstlane(*a.err)) return;  // this push already failed
+  spill_records(a, min(*a.ovf.count, (unsigned)a.ovf.cap), blockIdx.x * blockDim.x + threadIdx.x,
+                gridDim.x * blockDim.x);
 }
 
 // What the host wants to know of a push before it launches the next one, in
@@ -1069,16 +1097,13 @@ k_publish_push(const int* __restrict__ grp_rows, int ngroups, const int* err,
   publish_push(grp_rows, ngroups, err, ovf_count, seq, host);
 }
 
-// The field stages between the push and advance_e at one interior voxel (i, at
-// x, y, z): unload (src/accumulator.cpp:45-122), the J fold (k_fold_j's closed
-// form, from the accumulators directly: a voxel of the high ghost layer is
-// unloaded by the thread whose voxel it folds into) and advance_b with its
-// ghosts, in the order of the separate kernels for every value.  J is written
-// on interior voxels only: advance_e, which follows, writes the ghosts.
+// Unload (src/accumulator.cpp:45-122) and the J fold (k_fold_j's closed form,
+// from the accumulators directly: a voxel of the high ghost layer is unloaded by
+// the thread whose voxel it folds into) at one interior voxel (i, at x, y, z), in
+// the order of the separate kernels for every value.
 template <class R>
-__device__ __forceinline__ void currents_voxel(R* __restrict__ fields, const R* __restrict__ acc,
-                                               const Grid& g, int x, int y, int z, int i, R cx,
-                                               R cy, R cz, R px, R py, R pz) {
+__device__ __forceinline__ void currents_at(R* fields, const R* acc, const Grid& g, int x, int y,
+                                            int z, int i, R cx, R cy, R cz) {
   const size_t N = g.ncells;
   const int pos[3] = {x, y, z};
   const int n[3] = {g.nx, g.ny, g.nz};
@@ -1102,6 +1127,16 @@ __device__ __forceinline__ void currents_voxel(R* __restrict__ fields, const R* 
       J = J + unloaded(iq);
     fields[(6 + c) * N + i] = J;
   }
+}
+
+// The field stages between the push and advance_e at one interior voxel:
+// currents_at, then advance_b with its ghosts.  J is written on interior voxels
+// only: advance_e, which follows, writes the ghosts.
+template <class R>
+__device__ __forceinline__ void currents_voxel(R* __restrict__ fields, const R* __restrict__ acc,
+                                               const Grid& g, int x, int y, int z, int i, R cx,
+                                               R cy, R cz, R px, R py, R pz) {
+  currents_at(fields, acc, g, x, y, z, i, cx, cy, cz);
   advance_b_voxel(fields, g, x, y, z, i, px, py, pz);
 }
 
