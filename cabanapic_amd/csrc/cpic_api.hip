@@ -18,6 +18,7 @@
 #include "../../include/cabanapic_amd.h"
 #include "cpic_host_copy.h"
 #include "cpic_push_kernels.h"
+#include "cpic_block_kernels.h"
 #include "cpic_small_kernels.h"
 #include "cpic_split_kernels.h"
 #include "cpic_tangent_kernels.h"
@@ -361,23 +362,23 @@ void launch_arrive_split(cpic_context* c, const ArrivePass<R>& a, int S) {
          : k_arrive_split<R, K, 8><<<groups, 64 * 8, 0, c->stream>>>(a);
 }
 
-// push + move_p + deposit: pass 1, three finishing passes, spill fallback.
-// accumulate = 1 adds to the accumulators as the reference's push does;
-// accumulate = 0 overwrites them (valid right after a clear).  gather: where
-// pass 1 takes the interpolators from (the array, or the fields).
+// What the passes of one push are given.
+template <class R> struct PushArgs {
+  PushPass<R> push;
+  ArrivePass<R> arrive;
+  BlockFinish<R> finish;
+};
+
 template <class R>
-int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, int accumulate,
-               bool compact, int gather = kGatherRead) {
-  StageTimer t(c, CPIC_STAGE_PUSH);
-  if (c->np == 0) return t.finish();
-  if (c->D == 0) return fail(CPIC_ERR_INVALID, "particles resident without columns");
-  const int blocks = cdiv(c->nc, kBlock);
+PushArgs<R> push_args(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp,
+                      int accumulate, int gather) {
   Overflow<R> ovf{(R*)c->ovf_rec, c->ovf_cell, c->ovf_count, c->ovf_cap};
   RecordList<R> L1{(R*)c->rec1, c->rc1, c->M1, (int)c->nc};
   RecordList<R> L2{(R*)c->rec2, c->rc2, c->M2, (int)c->nc};
   const ColState<R> cs = col_state<R>(c, c->cur);
+  PushArgs<R> args;
 
-  PushPass<R> p;
+  PushPass<R>& p = args.push;
   p.cs = cs;
   p.dep = c->dep;
   p.dep_words = c->dep_words;
@@ -396,28 +397,9 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   p.err = c->err;
   p.grp_rows = c->grp_rows;
   p.grp_movers = c->grp_movers;
-  // k_push_split keeps every particle in its row; k_push_pass packs the
-  // columns.  The row stores of k_push_split address one column group with
-  // 32-bit byte offsets; columns too deep for that are packed at every push.
-  const bool group_fits = (int64_t)c->D * 64 * kSlotLen * (int64_t)sizeof(R) < INT32_MAX;
-  const SplitWaves waves = split_waves(c);
-  const bool small = small_grid(c);
-  const int cell_blocks = cdiv(c->nc, kSmallWaves);
-  const bool cells = small && !compact && group_fits;
-  c->n_movers = cells ? cell_blocks : column_groups(c);
-  if (cells)
-    c->compensated ? k_push_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p)
-                   : k_push_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p);
-  else if (compact || !group_fits)
-    c->compensated ? k_push_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
-                   : k_push_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
-  else
-    c->compensated ? launch_push_split<R, true>(c, p, waves.push)
-                   : launch_push_split<R, false>(c, p, waves.push);
-  CHECK_LAUNCH();
 
   // the streak after the 1st crossing, found through the departure masks
-  ArrivePass<R> ar;
+  ArrivePass<R>& ar = args.arrive;
   ar.cs = cs;
   ar.dep = c->dep;
   ar.dep_words = c->dep_words;
@@ -432,19 +414,12 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
   ar.cdt_dz = cdt_dz;
   ar.qsp = qsp;
   ar.err = c->err;
-  if (small)
-    c->compensated ? k_arrive_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar)
-                   : k_arrive_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar);
-  else
-    c->compensated ? launch_arrive_split<R, true>(c, ar, waves.arrive)
-                   : launch_arrive_split<R, false>(c, ar, waves.arrive);
-  CHECK_LAUNCH();
 
   // the streaks after the 2nd and 3rd crossings, from the record lists
   const RecordList<R> ins[2] = {L2, L1};
   const RecordList<R> outs[2] = {L1, L2};
   for (int pass = 0; pass < 2; ++pass) {
-    FinishPass<R> f;
+    FinishPass<R>& f = args.finish.pass[pass];
     f.cs = cs;
     f.in = ins[pass];
     f.out = outs[pass];
@@ -454,15 +429,69 @@ int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, 
     f.ncells = (int)c->ncells;
     f.qsp = qsp;
     f.last = (pass == 1) ? 1 : 0;
-    f.flag_set = (pass == 0) ? c->rec_flags : nullptr;
-    f.flag_skip = (pass == 1) ? c->rec_flags : nullptr;
+    f.flag_set = f.flag_skip = nullptr;
     f.err = c->err;
+  }
+  args.finish.spill = {cs, ovf, (R*)c->acc, c->cg, (int)c->ncells, qsp, c->err};
+  return args;
+}
+
+// The push's first two passes.
+template <class R>
+int launch_particle_passes(cpic_context* c, const PushArgs<R>& args, bool compact) {
+  const int blocks = cdiv(c->nc, kBlock);
+  // k_push_split keeps every particle in its row; k_push_pass packs the
+  // columns.  The row stores of k_push_split address one column group with
+  // 32-bit byte offsets; columns too deep for that are packed at every push.
+  const bool group_fits = (int64_t)c->D * 64 * kSlotLen * (int64_t)sizeof(R) < INT32_MAX;
+  const SplitWaves waves = split_waves(c);
+  const bool small = small_grid(c);
+  const int cell_blocks = cdiv(c->nc, kSmallWaves);
+  const bool cells = small && !compact && group_fits;
+  const PushPass<R>& p = args.push;
+  const ArrivePass<R>& ar = args.arrive;
+  c->n_movers = cells ? cell_blocks : column_groups(c);
+  if (cells)
+    c->compensated ? k_push_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p)
+                   : k_push_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p);
+  else if (compact || !group_fits)
+    c->compensated ? k_push_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
+                   : k_push_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
+  else
+    c->compensated ? launch_push_split<R, true>(c, p, waves.push)
+                   : launch_push_split<R, false>(c, p, waves.push);
+  CHECK_LAUNCH();
+  if (small)
+    c->compensated ? k_arrive_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar)
+                   : k_arrive_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(ar);
+  else
+    c->compensated ? launch_arrive_split<R, true>(c, ar, waves.arrive)
+                   : launch_arrive_split<R, false>(c, ar, waves.arrive);
+  CHECK_LAUNCH();
+  return CPIC_OK;
+}
+
+// push + move_p + deposit: pass 1, three finishing passes, spill fallback.
+// accumulate = 1 adds to the accumulators as the reference's push does;
+// accumulate = 0 overwrites them (valid right after a clear).  gather: where
+// pass 1 takes the interpolators from (the array, or the fields).
+template <class R>
+int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, int accumulate,
+               bool compact, int gather = kGatherRead) {
+  StageTimer t(c, CPIC_STAGE_PUSH);
+  if (c->np == 0) return t.finish();
+  if (c->D == 0) return fail(CPIC_ERR_INVALID, "particles resident without columns");
+  const int blocks = cdiv(c->nc, kBlock);
+  PushArgs<R> args =
+      push_args<R>(c, qdt_2mc, cdt_dx, cdt_dy, cdt_dz, qsp, accumulate, gather);
+  if (int s = launch_particle_passes<R>(c, args, compact)) return s;
+  args.finish.pass[0].flag_set = args.finish.pass[1].flag_skip = c->rec_flags;
+  for (const FinishPass<R>& f : args.finish.pass) {
     c->compensated ? k_finish_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(f)
                    : k_finish_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(f);
     CHECK_LAUNCH();
   }
-  SpillPass<R> sp{cs, ovf, (R*)c->acc, c->cg, (int)c->ncells, qsp, c->err};
-  k_spill_pass<R><<<64, kBlock, 0, c->stream>>>(sp);
+  k_spill_pass<R><<<64, kBlock, 0, c->stream>>>(args.finish.spill);
   CHECK_LAUNCH();
   c->cur = 1 - c->cur;
   return t.finish();
@@ -928,6 +957,44 @@ int stage_fields(cpic_context* c, const cpic_step_params* sp, int erow) {
   return CPIC_OK;
 }
 
+template <class R>
+BlockTail<R> block_tail(cpic_context* c, const cpic_step_params* sp, const PushArgs<R>& args,
+                        double* row) {
+  const R px = (R)sp->px, py = (R)sp->py, pz = (R)sp->pz;
+  const R half = (R)0.5;
+  R cx, cy, cz;
+  unload_scales<R>((R)sp->dx, (R)sp->dy, (R)sp->dz, (R)sp->dt, cx, cy, cz);
+  next_status(c);
+  return {args.finish,
+          {(R*)c->fields, (const R*)c->acc, c->grid, cx, cy, cz, half * px, half * py, half * pz,
+           px, py, pz, (R)sp->dt_eps0},
+          {c->grp_rows, column_groups(c), c->err, c->ovf_count, c->push_seq, c->push_host},
+          row};
+}
+
+// Whether the stages after the particle passes run in one workgroup.
+bool tail_in_block(const cpic_context* c) { return c->nc <= kBlockThreads; }
+
+template <class R>
+PushArgs<R> step_args(cpic_context* c, const cpic_step_params* sp, int gather) {
+  return push_args<R>(c, (R)sp->qdt_2mc, (R)sp->cdt_dx, (R)sp->cdt_dy, (R)sp->cdt_dz,
+                      (R)sp->qsp, 0, gather);
+}
+
+// One step with the stages after the particle passes in one launch.
+template <class R>
+int launch_tail_step(cpic_context* c, const cpic_step_params* sp, int gather, bool compact,
+                     double* row) {
+  const PushArgs<R> args = step_args<R>(c, sp, gather);
+  if (int s = launch_particle_passes<R>(c, args, compact)) return s;
+  const BlockTail<R> tail = block_tail<R>(c, sp, args, row);
+  c->compensated ? k_block_tail<R, true><<<1, kBlockThreads, 0, c->stream>>>(tail)
+                 : k_block_tail<R, false><<<1, kBlockThreads, 0, c->stream>>>(tail);
+  CHECK_LAUNCH();
+  c->cur = 1 - c->cur;
+  return CPIC_OK;
+}
+
 // nsteps iterations of the loop body of example/example.cpp:216-279 on the
 // context's stream, no host synchronisation; energies of step s (1-based)
 // into dhist row s - 1 (3 doubles: E, B, kinetic) when dhist is not null,
@@ -944,6 +1011,7 @@ int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, doubl
                          (1u << CPIC_STAGE_ADVANCE_E) | (1u << CPIC_STAGE_ENERGY);
   const bool fuse_fields =
       c->solver == CPIC_FIELD_SOLVER_EM && !(c->timing & timed) && c->np > 0 && c->D > 0;
+  const bool tail = fuse_fields && !c->timing && tail_in_block(c);
   const int eblocks = cdiv(c->nc, kBlock);
   int erows = 0;  // sets of energy partials waiting to be summed
   for (int64_t step = 1; step <= nsteps; ++step) {
@@ -957,14 +1025,19 @@ int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, doubl
     // needed while ghost accumulators may hold data
     if (!c->acc_ghosts_zero && (t = stage_clear<R>(c))) return t;
     if ((t = check_headroom(c))) return t;
-    const bool compact = packs_now(c, sp->compact_interval);
-    const int gather = !fused ? kGatherRead : step == nsteps ? kGatherStore : kGatherFields;
-    if ((t = stage_push<R>(c, (R)sp->qdt_2mc, (R)sp->cdt_dx, (R)sp->cdt_dy, (R)sp->cdt_dz,
-                           (R)sp->qsp, 0, compact, gather)))
-      return t;
     const bool do_e = ei > 0 && step % ei == 0, do_k = ki > 0 && step % ki == 0;
     double* row = dhist ? dhist + 3 * (step - 1) : c->red_out;
-    if (fuse_fields) {
+    const bool compact = packs_now(c, sp->compact_interval);
+    const int gather = !fused ? kGatherRead : step == nsteps ? kGatherStore : kGatherFields;
+    if (tail) {
+      if ((t = launch_tail_step<R>(c, sp, gather, compact, do_e ? row : nullptr))) return t;
+    } else if ((t = stage_push<R>(c, (R)sp->qdt_2mc, (R)sp->cdt_dx, (R)sp->cdt_dy,
+                                  (R)sp->cdt_dz, (R)sp->qsp, 0, compact, gather))) {
+      return t;
+    }
+    if (tail) {
+      // done
+    } else if (fuse_fields) {
       if ((t = stage_fields<R>(c, sp, do_e ? erows : -1))) return t;
       // the partials of many steps are summed by one launch (without a
       // history, each step's into the same place: the last energies are kept)
