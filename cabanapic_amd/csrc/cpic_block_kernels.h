@@ -6,8 +6,8 @@
 // at most a thread per cell.  On a 1D deck they took 21 of a step's 50 us: each
 // launch starts with cold caches and drains before the next.  Up to
 // kBlockThreads cells one workgroup runs them all, with barriers in the
-// launches' places: 13.5 us for 32 cells, a step 50 -> 46 us in FP64 and, with
-// a dump of the particles after every step, 71 -> 58 in FP32.  Every value is
+// launches' places: 11 us for 32 cells, and a step, with the push's status sent
+// to the host before the field stages, 50 -> 40 us in FP64.  Every value is
 // computed by the same operations, and every sum in the same order, as in the
 // kernels that larger grids run.
 //
@@ -235,13 +235,14 @@ __global__ void __launch_bounds__(kBlockThreads) k_block_tail(BlockTail<R>) {
   }
   __syncthreads();
   if (!__builtin_amdgcn_readfirstlane(failed)) block_finish<R, K>(crossed);
+  // before the field stages: the host may be waiting for it to queue the next step
+  const BlockStatus& status = phase_args<R>().status;
+  if (threadIdx.x >= kBlockThreads - 64) block_publish(status, threadIdx.x & 63);
   const bool energy = phase_args<R>().row != nullptr;
   block_fields<R>(energy, sums);
   __syncthreads();
-  const BlockTail<R>& a = phase_args<R>();
-  const int t = threadIdx.x;
-  if (energy && t == 0) block_energies(sums, a.row);
-  if (t >= kBlockThreads - 64) block_publish(a.status, t & 63);
+  double* const row = phase_args<R>().row;
+  if (energy && threadIdx.x == 0) block_energies(sums, row);
 }
 
 }  // namespace cpic
