@@ -94,8 +94,19 @@ template <class R, bool K, int S> struct RowSums {
     else
       __syncthreads();
   }
-  // the sums to (or onto) the accumulators of voxel v
-  __device__ __forceinline__ void store(R* acc, size_t N, int v, int wave, bool onto) const {
+  // the accumulators of voxel v that the wave's sums go to
+  __device__ __forceinline__ void fetch(const R* acc, size_t N, int v, int wave,
+                                        R (&was)[kQuads][4]) const {
+#pragma unroll
+    for (int i = 0; i < kQuads; ++i) {
+      const int q = wave + i * S;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) was[i][k] = q < 3 ? acc[(size_t)(4 * q + k) * N + v] : 0;
+    }
+  }
+  // the sums to the accumulators, or onto what they hold, was
+  __device__ __forceinline__ void store(R* acc, size_t N, int v, int wave, bool onto,
+                                        const R (&was)[kQuads][4]) const {
 #pragma unroll
     for (int i = 0; i < kQuads; ++i) {
       const int q = wave + i * S;
@@ -103,8 +114,7 @@ template <class R, bool K, int S> struct RowSums {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const R t = K ? s[i][k] + c[K ? i : 0][k] : s[i][k];
-          R* p = acc + (size_t)(4 * q + k) * N + v;
-          *p = onto ? *p + t : t;
+          acc[(size_t)(4 * q + k) * N + v] = onto ? was[i][k] + t : t;
         }
       }
     }
@@ -228,7 +238,11 @@ __global__ void __launch_bounds__(64 * S) k_push_split(PushPass<R> a) {
     }
   }
   for (int w = nwords + wave; w < MW; w += S) a.cs.mask_out[(size_t)w * MP + ci] = 0ull;
-  if (valid) sums.store(a.acc, a.ncells, v, wave, a.accumulate);
+  if (valid) {
+    R was[Sums::kQuads][4] = {};
+    if (a.accumulate) sums.fetch(a.acc, a.ncells, v, wave, was);
+    sums.store(a.acc, a.ncells, v, wave, a.accumulate, was);
+  }
   const int wm = wave_sum_int(nmov);
   if (lane == 0) movers[wave] = wm;
   __syncthreads();
@@ -332,6 +346,17 @@ __global__ void __launch_bounds__(64 * S) k_arrive_split(ArrivePass<R> a) {
   const unsigned long long* const occ = a.cs.mask_out + ci;
   const unsigned long long occ0 = *occ;
   int len = min(a.cs.cnt_out[ci], a.cs.D);  // rows in use (kept by wave 0)
+  // and what the end of the pass updates: the wave's first word, and its sums
+  // (where two waves share a group they are six quads a lane, whose registers
+  // would cost FP64 a third of the waves, on grids that hide the latency anyway)
+  constexpr bool kFetchEarly = S > 2;
+  Sums sums;
+  R was[Sums::kQuads][4];
+  if (kFetchEarly) sums.fetch(a.acc, a.ncells, v, wave, was);
+  const int w1 = min(wave, MW - 1);
+  const unsigned long long occ1 = occ[(size_t)w1 * MP];
+  const unsigned long long own1 = a.dep[dep_index(6, w1, MW, MP, ci)];
+  const int own_words = min(a.dep_words[grp], MW);
   // one look at the flags for the block: a wave of this launch may raise one
   // meanwhile, and all waves must reach the same barriers
   if (threadIdx.x == 0) failed = *a.err;
@@ -344,7 +369,6 @@ __global__ void __launch_bounds__(64 * S) k_arrive_split(ArrivePass<R> a) {
   }
   __syncthreads();
   if (failed) return;
-  Sums sums;
   sums.zero();
   FreeRows rows;
   rows.start(occ0, a.cs.D);
@@ -464,16 +488,19 @@ __global__ void __launch_bounds__(64 * S) k_arrive_split(ArrivePass<R> a) {
   // free: other lanes may still be reading those rows in this pass, but nobody
   // writes them before the next one, which is the first that can hand them out
   // again
-  const int own_words = min(a.dep_words[grp], MW);
   for (int w = wave; w < MW; w += S) {
     const unsigned long long add = w < kTakenWords ? taken[w][lane] : deep[(size_t)w * MP];
-    const unsigned long long own = w < own_words ? a.dep[dep_index(6, w, MW, MP, ci)] : 0ull;
+    const unsigned long long own =
+        w >= own_words ? 0ull : w == wave ? own1 : a.dep[dep_index(6, w, MW, MP, ci)];
     if (add | own) {
       unsigned long long* m = a.cs.mask_out + (size_t)w * MP + ci;
-      *m = (*m | add) & ~own;
+      *m = ((w == wave ? occ1 : *m) | add) & ~own;
     }
   }
-  if (any) sums.store(a.acc, a.ncells, v, wave, true);
+  if (any) {
+    if (!kFetchEarly) sums.fetch(a.acc, a.ncells, v, wave, was);
+    sums.store(a.acc, a.ncells, v, wave, true, was);
+  }
   if (wave != 0) return;
   a.cs.cnt_out[ci] = len;
 #pragma unroll
