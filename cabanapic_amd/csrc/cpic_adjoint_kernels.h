@@ -35,8 +35,10 @@ namespace cpic {
 // w, tag), with the interior cell of every slot; first[ci] = position of
 // cell ci's first particle, first[nc] = n.
 
-// Exclusive prefix sum of cnt[0..n) into out[0..n], out[n] = total, in three
-// passes (block scans, a scan of the block totals, the block offsets added).
+// Exclusive prefix sum of n counts into out[0..n], out[n] = total, in two
+// passes: block scans, then every block adds the totals of the blocks before it,
+// which it sums itself.  (With the counts' own launch and one that scans the
+// totals they were four, of 4 us each on small grids.)
 constexpr int kScanItems = 8;  // elements per thread of a block scan
 
 __device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
@@ -61,13 +63,29 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
   return before + x - v;
 }
 
+// Count i of an array.
+struct ArrayCounts {
+  const int* in;
+  __device__ __forceinline__ int operator()(int i) const { return in[i]; }
+};
+// Particles of cell i's column.
+struct ColumnCounts {
+  const int* cnt;
+  const unsigned long long* mask;
+  int nc_pad, D;
+  __device__ __forceinline__ int operator()(int i) const {
+    return column_occupancy(cnt, mask, nc_pad, D, i);
+  }
+};
+
+template <class Counts>
 __global__ void __launch_bounds__(kBlock)
-k_scan_blocks(const int* __restrict__ in, int n, int* __restrict__ out, int* __restrict__ sums) {
+k_scan_blocks(Counts count, int n, int* out, int* __restrict__ sums) {
   const int base = blockIdx.x * kBlock * kScanItems + threadIdx.x * kScanItems;
   int v[kScanItems], s = 0;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
-    v[k] = base + k < n ? in[base + k] : 0;
+    v[k] = base + k < n ? count(base + k) : 0;
     s += v[k];
   }
   int total;
@@ -80,28 +98,17 @@ k_scan_blocks(const int* __restrict__ in, int n, int* __restrict__ out, int* __r
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// one block: exclusive scan of the nb block sums in place, grand total to *total_out
-__global__ void __launch_bounds__(kBlock) k_scan_sums(int* __restrict__ sums, int nb,
-                                                      int* __restrict__ total_out) {
-  int carry = 0;
-  for (int b0 = 0; b0 < nb; b0 += kBlock) {
-    const int i = b0 + threadIdx.x;
-    const int v = i < nb ? sums[i] : 0;
-    int total;
-    const int ex = block_exclusive_scan(v, &total);
-    if (i < nb) sums[i] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) *total_out = carry;
-}
-
 __global__ void __launch_bounds__(kBlock)
 k_scan_add(int* __restrict__ out, int n, const int* __restrict__ sums) {
+  int part = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) part += sums[b];
+  int add;
+  (void)block_exclusive_scan(part, &add);
   const int base = blockIdx.x * kBlock * kScanItems + threadIdx.x * kScanItems;
-  const int add = sums[blockIdx.x];
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k)
     if (base + k < n) out[base + k] += add;
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = add + sums[blockIdx.x];
 }
 
 // The position of set bit n (from 0) of m, which has more.
@@ -129,8 +136,17 @@ template <class R>
 __global__ void __launch_bounds__(kSnapBlock)
 k_snapshot_columns(const R* __restrict__ cols, const int* __restrict__ cnt,
                    const unsigned long long* __restrict__ mask, int nc, int nc_pad, int D,
-                   const int* __restrict__ first, R* __restrict__ slots, int* __restrict__ cell) {
+                   const int* __restrict__ first, R* __restrict__ slots, int* __restrict__ cell,
+                   const R* __restrict__ fields, R* __restrict__ kept_fields, size_t nf) {
   typedef typename Vec4T<R>::type V4;
+  // the blocks past the groups' copy the fields
+  const int groups = nc_pad / 64;
+  if ((int)blockIdx.x >= groups) {
+    const size_t stride = (size_t)(gridDim.x - groups) * kSnapBlock;
+    for (size_t i = (size_t)(blockIdx.x - groups) * kSnapBlock + threadIdx.x; i < nf; i += stride)
+      kept_fields[i] = fields[i];
+    return;
+  }
   __shared__ int start[65], rows[64];
   __shared__ unsigned long long occ[64];  // the first mask words
   const int c0 = blockIdx.x * 64;

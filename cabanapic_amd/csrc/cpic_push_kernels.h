@@ -1390,17 +1390,21 @@ k_masks_packed(const int* __restrict__ cnt, unsigned long long* __restrict__ mas
   for (int w = 0; w < MW; ++w) mask[(size_t)w * nc_pad + ci] = low_bits(n - 64 * w);
 }
 
-// Particles held by each cell (occupied rows below its count).
-__global__ void __launch_bounds__(kBlock)
-k_column_occupancy(const int* __restrict__ cnt, const unsigned long long* __restrict__ mask,
-                   int nc, int nc_pad, int D, int* __restrict__ occ) {
-  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
-  if (ci >= nc) return;
+// Particles held by cell ci (occupied rows below its count).
+__device__ __forceinline__ int column_occupancy(const int* cnt, const unsigned long long* mask,
+                                                int nc_pad, int D, int ci) {
   const int n = min(cnt[ci], D);
   int k = 0;
   for (int w = 0; 64 * w < n; ++w)
     k += __popcll(mask[(size_t)w * nc_pad + ci] & low_bits(n - 64 * w));
-  occ[ci] = k;
+  return k;
+}
+
+__global__ void __launch_bounds__(kBlock)
+k_column_occupancy(const int* __restrict__ cnt, const unsigned long long* __restrict__ mask,
+                   int nc, int nc_pad, int D, int* __restrict__ occ) {
+  const int ci = blockIdx.x * blockDim.x + threadIdx.x;
+  if (ci < nc) occ[ci] = column_occupancy(cnt, mask, nc_pad, D, ci);
 }
 
 // Download: the particles of cell ci, occupied rows in row order, go to
