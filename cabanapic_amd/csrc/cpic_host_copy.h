@@ -4,8 +4,15 @@
 // been allocated (one thread moves the data out of a staging buffer and takes
 // the page faults): 7.9 ms for the 79 MB of fields of a 128^3 grid, an eighth
 // of 24 steps.  Here the copy engine fills 2 MB pieces of a pinned ring while
-// four threads empty it: 2.2 ms (36 GB/s; 10 MB 0.99 -> 0.46 ms, 50 MB 5.0 ->
-// 1.5 ms).  1 MB pieces reach 29 GB/s, one thread 14, six threads no more.
+// up to four threads empty it: 2.2 ms (36 GB/s; 50 MB 5.0 -> 1.5 ms).  1 MB
+// pieces reach 29 GB/s, one thread 14, six threads no more.
+//
+// The caller is one of the threads, and the only one below 16 MB, where others
+// gain little (7 MB 0.45 against 0.5 ms) and cost much where the program's own
+// threads, spinning after a parallel loop, use up the process's CPUs: gradients of
+// 25x25x15 x 15 particles, whose owner rounds them with such a loop, took 1.8 or
+// 4 ms a pass with four threads beside the caller, 1.8 always with the caller
+// alone.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -79,70 +86,61 @@ class HostRing {
     return ring_ != nullptr;
   }
 
+  // Threads that empty the ring, the caller among them (each divides kPieces).
+  static int threads_for(size_t n) { return n < (16u << 20) ? 1 : n < (32u << 20) ? 2 : kThreads; }
+
+  // Piece i goes through slot i % kPieces and is thread i % threads's, which
+  // empties the slot and then has the copy engine fill it with the next piece of
+  // the slot, its own too: the threads share nothing but the stream.
   hipError_t ringed(char* dst, const char* src, size_t n, hipStream_t stream) {
     const long pieces = (long)((n + kPiece - 1) / kPiece);
-    auto size = [&](long i) { return std::min(kPiece, n - (size_t)i * kPiece); };
-    std::vector<std::thread> pool;
-    pool.reserve(kThreads);
+    const int threads = threads_for(n);
     hipEvent_t ev[kPieces] = {};
     int device = 0;
     hipError_t err = hipGetDevice(&device);
     for (int k = 0; k < kPieces && err == hipSuccess; ++k)
       err = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-    // piece i is in slot i % kPieces; queued: pieces handed to the copy engine,
-    // emptied[t]: pieces that thread t (i % threads == t) has copied out.  A
-    // piece is counted whatever became of it, so that nobody waits for ever.
-    std::atomic<long> queued{0};
-    std::atomic<long> emptied[kThreads];
-    for (auto& e : emptied) e = 0;
-    std::atomic<int> failure{(int)hipSuccess};
+    std::atomic<int> failure{(int)err};
+    auto size = [&](long i) { return std::min(kPiece, n - (size_t)i * kPiece); };
+    auto slot = [&](long i) { return ring_ + (size_t)(i % kPieces) * kPiece; };
+    auto fill = [&](long i) {
+      hipError_t e = hipMemcpyAsync(slot(i), src + (size_t)i * kPiece, size(i),
+                                    hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipEventRecord(ev[i % kPieces], stream);
+      if (e != hipSuccess) failure = (int)e;
+    };
     auto empty = [&](int t) {
-      (void)hipSetDevice(device);
-      for (long i = t; i < pieces; i += kThreads) {
-        while (queued.load(std::memory_order_acquire) <= i) std::this_thread::yield();
-        if (failure.load() == (int)hipSuccess) {
-          const hipError_t e = hipEventSynchronize(ev[i % kPieces]);
-          if (e == hipSuccess)
-            memcpy(dst + (size_t)i * kPiece, ring_ + (size_t)(i % kPieces) * kPiece, size(i));
-          else
-            failure = (int)e;
+      for (long i = t; i < pieces && failure == (int)hipSuccess; i += threads) {
+        const hipError_t e = hipEventSynchronize(ev[i % kPieces]);
+        if (e != hipSuccess) {
+          failure = (int)e;
+          return;
         }
-        emptied[t].fetch_add(1, std::memory_order_release);
+        memcpy(dst + (size_t)i * kPiece, slot(i), size(i));
+        if (i + kPieces < pieces) fill(i + kPieces);
       }
     };
-    if (err == hipSuccess) {
-      try {
-        for (int t = 0; t < kThreads; ++t) pool.emplace_back(empty, t);
-      } catch (...) {
-        // no threads to be had: those that started are let run dry
-        failure = (int)hipErrorOutOfMemory;
-        queued = pieces;
-        for (auto& th : pool) th.join();
-        for (hipEvent_t e : ev) (void)hipEventDestroy(e);
-        return plain(dst, src, n, stream);
-      }
-      for (long i = 0; i < pieces; ++i) {
-        const long before = i - kPieces;  // the piece that had the slot
-        if (before >= 0)
-          while (emptied[before % kThreads].load(std::memory_order_acquire) <= before / kThreads)
-            std::this_thread::yield();
-        if (failure.load() == (int)hipSuccess) {
-          hipError_t e = hipMemcpyAsync(ring_ + (size_t)(i % kPieces) * kPiece,
-                                        src + (size_t)i * kPiece, size(i), hipMemcpyDeviceToHost,
-                                        stream);
-          if (e == hipSuccess) e = hipEventRecord(ev[i % kPieces], stream);
-          if (e != hipSuccess) failure = (int)e;
-        }
-        queued.store(i + 1, std::memory_order_release);
-      }
-      for (auto& th : pool) th.join();
-      err = (hipError_t)failure.load();
+    for (long i = 0; i < std::min<long>(pieces, kPieces) && failure == (int)hipSuccess; ++i) fill(i);
+    std::vector<std::thread> pool;
+    int started = 1;
+    try {
+      pool.reserve(threads);
+      for (; started < threads; ++started)
+        pool.emplace_back([&, t = started] {
+          (void)hipSetDevice(device);
+          empty(t);
+        });
+    } catch (...) {
+      // no more threads to be had: the caller takes their pieces
     }
+    empty(0);
+    for (int t = started; t < threads; ++t) empty(t);
+    for (auto& th : pool) th.join();
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
     // (after a failure copies into the ring may still be in flight)
-    if (err != hipSuccess) (void)hipStreamSynchronize(stream);
-    return err;
+    if (failure != (int)hipSuccess) (void)hipStreamSynchronize(stream);
+    return (hipError_t)failure.load();
   }
 };
 
