@@ -496,11 +496,52 @@ template <class R> struct TangentFields {
   Grid g;
 };
 
-// load_interpolator_array and clear_accumulator_array, one thread per voxel.
+// Where the energies of the last step go: one block sums the partials (E, B,
+// E . tE, B . tB) that its k_tangent_advance_b left in nblocks sets.
+struct TangentRow {
+  const double* partials;
+  int nblocks;
+  double* hist;  // null: no history
+  int* counter;  // steps begun since the call began (on the device: a graph's arguments
+                 // cannot change from step to step)
+  int cap;       // rows of hist
+};
+
+__device__ __forceinline__ void tangent_row(const TangentRow& a) {
+  double v[4] = {0, 0, 0, 0};
+  for (int b = threadIdx.x; b < a.nblocks; b += blockDim.x)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] += a.partials[(size_t)b * 4 + q];
+  __shared__ double res[4];
+  block_sum_store<4>(v, res);
+  if (threadIdx.x != 0) return;
+  const int r = *a.counter;
+  *a.counter = r + 1;
+  if (r < 1 || r > a.cap) return;  // no step before, or no row for it
+  double* const row = a.hist + 4 * (size_t)(r - 1);
+  row[0] = 0.5 * res[0];
+  row[1] = 0.5 * res[1];
+  row[2] = res[2];
+  row[3] = res[3];
+}
+
+// The row of the call's last step.
+__global__ void __launch_bounds__(kBlock) k_tangent_row(TangentRow a) { tangent_row(a); }
+
+// load_interpolator_array and clear_accumulator_array, one thread per voxel,
+// which also clears its bin of the sort that follows (bins not null).  One block
+// more with a history: the energies of the step before, whose own launch took
+// 4 us of a 32^3 step's 150.
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_tangent_begin(TangentFields<R> a) {
+__global__ void __launch_bounds__(kBlock)
+k_tangent_begin(TangentFields<R> a, TangentRow last, int* __restrict__ bins) {
+  if (last.hist && blockIdx.x == gridDim.x - 1) {
+    tangent_row(last);
+    return;
+  }
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const Grid& g = a.g;
+  if (bins && i <= g.ncells) bins[i] = 0;
   if (i >= g.ncells) return;
   const size_t N = g.ncells;
 #pragma unroll
@@ -578,28 +619,6 @@ k_tangent_advance_b(TangentFields<R> a, R px, R py, R pz, double tpx, double tpy
     }
   }
   block_sum_store<4>(v, partials + 4 * (size_t)blockIdx.x);
-}
-
-// One block: the step's row (E, B, dE, dB) from those sums, to the history row
-// that a device counter names (a graph's arguments cannot change from step to
-// step); the counter moves on.
-__global__ void __launch_bounds__(kBlock)
-k_tangent_row(const double* __restrict__ partials, int nblocks, double* __restrict__ hist,
-              int* __restrict__ counter, int cap) {
-  double v[4] = {0, 0, 0, 0};
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] += partials[(size_t)b * 4 + q];
-  __shared__ double res[4];
-  block_sum_store<4>(v, res);
-  if (threadIdx.x != 0) return;
-  const int r = *counter;
-  *counter = r + 1;
-  if (r >= cap) return;
-  hist[4 * (size_t)r] = 0.5 * res[0];
-  hist[4 * (size_t)r + 1] = 0.5 * res[1];
-  hist[4 * (size_t)r + 2] = res[2];
-  hist[4 * (size_t)r + 3] = res[3];
 }
 
 // sum over interior cells of E . tE and B . tB -> partials[block][2] (FP64):
