@@ -326,18 +326,24 @@ SplitWaves split_waves(const cpic_context* c) {
 }
 
 // Whether the kernels for grids of few cells run: a wave per cell instead of a
-// lane, for up to 4096 cells, whose waves find the chip's 256 CUs mostly idle.
-// A step in us, a wave per cell / a lane, two-stream plasmas in FP32 and FP64:
+// lane, for up to 4096 cells, whose waves find the chip's 256 CUs mostly idle,
+// and up to 8192 of enough particles to fill the waves' lanes.  A step in us, a
+// wave per cell / a lane (Weibel plasmas; the first three two-stream plasmas in
+// 1D, their figures before the loads of both passes were issued together):
 //   cells x particles     FP32          FP64
 //   32 x 64               42 / 62       45 / 81
 //   200 x 200             63 / 159      67 / 220
 //   1000 x 16             38 / 46       40 / 53
-//   12^3 x 64             59 / 87       65 / 108
-//   16^3 x 16             52 / 58       57 / 67
-//   16^3 x 200            96 / 170      118 / 212
-//   20^3 x 16             65 / 61       73 / 69
-//   24^3 x 64             114 / 94      149 / 124
-bool small_grid(const cpic_context* c) { return c->nc <= kSmallCells; }
+//   18^3 x 8              50 / 49       58 / 53
+//   18^3 x 24             56 / 59       64 / 66
+//   18^3 x 64             63 / 84       74 / 98
+//   20^3 x 8              55 / 50       65 / 54
+//   20^3 x 24             61 / 60       72 / 67
+//   20^3 x 64             69 / 84       83 / 100
+//   24^3 x 64             87 / 86       113 / 104
+bool small_grid(const cpic_context* c) {
+  return c->nc <= kSmallCells || (c->nc <= 2 * kSmallCells && c->np >= 32 * c->nc);
+}
 
 // Whether this push packs the columns: every interval-th one that the caller
 // names, by default every kCompactInterval-th of a grid that fills the chip.

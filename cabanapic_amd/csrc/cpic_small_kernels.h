@@ -5,7 +5,7 @@
 // cells of 64 particles in FP64, 26 in pass 2.  Here the roles are swapped: a
 // wave owns one cell, its lanes the rows (pass 1) or the arrivals (pass 2) of
 // that cell, so that a column of 64 particles takes one particle's time and
-// the cells spread over the chip: 11.7 and 13.4 us.  The contributions meet in
+// the cells spread over the chip: 10.5 and 7.5 us.  The contributions meet in
 // LDS and are added in row (arrival) order, so every result has the bits of
 // the other kernels'.
 #pragma once
@@ -16,7 +16,7 @@ namespace cpic {
 
 constexpr int kSmallWaves = 4;      // cells per block: a 128-byte line of FP32 slots
 constexpr int kSmallWords = 64;     // mask words whose taken rows k_arrive_cells notes in LDS
-constexpr int kSmallCells = 4096;   // cells of a grid that uses them
+constexpr int kSmallCells = 4096;   // cells of a grid that uses them in any case
 
 // Contributions of up to 64 rows, [12][rows], and the sums of the cell: lane
 // k < 12 of the wave holds sum k.  The padding puts the lanes' reads of four

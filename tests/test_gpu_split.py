@@ -2,7 +2,7 @@
 per cell, at the sizes where they can go wrong: groups of 64 cells that are
 partly filled, columns around a mask word and past what one chunk of words
 holds, columns too deep for LDS, both wave counts (up to 512 groups of cells, and more), 4096 cells and
-4097, more arrivals than lanes, and steps without some of the energies.  Particles equal the oracle's bit for bit;
+4097, 8192 of 31 and 32 particles and 8193, more arrivals than lanes, and steps without some of the energies.  Particles equal the oracle's bit for bit;
 accumulators agree within the bound of a reordered sum (as in
 test_gpu_parity.py)."""
 import numpy as np
@@ -22,6 +22,8 @@ CASES = [
     (16, 16, 16, 9, 0, 2), (241, 17, 1, 9, 0, 2), (3, 2, 1, 900, 0, 3),
     (63, 1, 1, 3, 4200, 3), (3, 1, 1, 1500, 0, 3), (241, 17, 1, 1, 0, 3),
     (241, 17, 1, 65, 0, 2), (241, 17, 1, 300, 0, 2),
+    (64, 16, 8, 31, 0, 2), (64, 16, 8, 32, 0, 2), (2731, 3, 1, 32, 0, 2), (2731, 3, 1, 65, 0, 2),
+    (2731, 3, 1, 300, 0, 2),
 ]
 
 
