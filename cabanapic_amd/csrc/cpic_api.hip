@@ -109,8 +109,9 @@ struct ColumnSet {
   int* grp_rows = nullptr;
   int* grp_movers = nullptr;
   int n_movers = 0;
-  // rows that pass 2 took, [MW][nc_pad], for columns of more than
-  // kTakenWords words only (kSmallWords is more)
+  // rows that pass 2 took, [MW][nc_pad], only for columns of more mask words
+  // than it notes in LDS: kTakenWords, or kSmallWords where k_arrive_cells runs
+  // whatever the particles' number
   unsigned long long* taken = nullptr;
 };
 
@@ -675,7 +676,7 @@ int alloc_column_set(cpic_context* c, int D, int M1, int M2, ColumnSet& out) {
     // (movers: k_push_cells counts per block of kSmallWaves cells)
     const size_t ints = 3 * groups + (size_t)c->nc_pad / kSmallWaves;
     if ((t = alloc((void**)&s.dep_words, sizeof(int) * ints))) return t;
-    if (s.MW > kTakenWords)
+    if (s.MW > (c->nc <= kSmallCells ? kSmallWords : kTakenWords))
       if ((t = alloc((void**)&s.taken, sizeof(unsigned long long) * words))) return t;
     s.rec_flags = s.dep_words + groups;
     s.grp_rows = s.dep_words + 2 * groups;
