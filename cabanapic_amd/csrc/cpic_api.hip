@@ -457,11 +457,14 @@ int launch_particle_passes(cpic_context* c, const PushArgs<R>& args, bool compac
   const bool cells = small && !compact && group_fits;
   const PushPass<R>& p = args.push;
   const ArrivePass<R>& ar = args.arrive;
-  c->n_movers = cells ? cell_blocks : column_groups(c);
+  const bool packs = compact || !group_fits;
+  // the counts that the launch below writes: entries past them are an earlier
+  // push's (another kernel's, if the number of particles has changed since)
+  c->n_movers = cells ? cell_blocks : packs ? column_groups(c) : cdiv(c->nc, 64);
   if (cells)
     c->compensated ? k_push_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p)
                    : k_push_cells<R, false><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p);
-  else if (compact || !group_fits)
+  else if (packs)
     c->compensated ? k_push_pass<R, true><<<blocks, kBlock, 0, c->stream>>>(p)
                    : k_push_pass<R, false><<<blocks, kBlock, 0, c->stream>>>(p);
   else
