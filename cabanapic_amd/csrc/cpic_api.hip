@@ -105,10 +105,8 @@ struct ColumnSet {
   // second, whose waves without a mark have nothing to do
   int* rec_flags = nullptr;
   // in the same allocation: per group the rows its columns used in the last
-  // push, and the particles that took the move_p branch, in n_movers counts
+  // push
   int* grp_rows = nullptr;
-  int* grp_movers = nullptr;
-  int n_movers = 0;
   // rows that pass 2 took, [MW][nc_pad], only for columns of more mask words
   // than it notes in LDS: kTakenWords, or kSmallWords where k_arrive_cells runs
   // whatever the particles' number
@@ -138,7 +136,7 @@ struct cpic_context : ColumnSet {
                            // compaction interval packs the columns)
   // device status words, one allocation (status), each on its own 256-byte
   // line: [0] error flags (err), [kStatusStride] overflow records (ovf_count,
-  // zero between pushes)
+  // zero between pushes); then cell_movers
   int* status = nullptr;
   unsigned int* ovf_count = nullptr;
 
@@ -151,8 +149,12 @@ struct cpic_context : ColumnSet {
   int partial_rows = 1;
   double* red_out = nullptr;   // [E, B, KE]
   int* err = nullptr;
-  int* block_movers = nullptr;  // movers of the last tangent push, per block (not owned)
-  int n_block_movers = 0;
+  // particles that took the move_p branch in a push, counted per group or block
+  // of cells (in status; the count outlives the columns), and the counts of the
+  // last push: those, or a tangent push's per block (not owned)
+  int* cell_movers = nullptr;
+  const int* last_movers = nullptr;
+  int n_movers = 0;
   double* hist_dev = nullptr;  // per-step energy rows of cpic_step
   long hist_cap = 0;           // rows allocated in hist_dev
   int n_partials = 0;
@@ -403,7 +405,7 @@ PushArgs<R> push_args(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, 
   p.accumulate = accumulate;
   p.err = c->err;
   p.grp_rows = c->grp_rows;
-  p.grp_movers = c->grp_movers;
+  p.grp_movers = c->cell_movers;
 
   // the streak after the 1st crossing, found through the departure masks
   ArrivePass<R>& ar = args.arrive;
@@ -460,6 +462,7 @@ int launch_particle_passes(cpic_context* c, const PushArgs<R>& args, bool compac
   const bool packs = compact || !group_fits;
   // the counts that the launch below writes: entries past them are an earlier
   // push's (another kernel's, if the number of particles has changed since)
+  c->last_movers = c->cell_movers;
   c->n_movers = cells ? cell_blocks : packs ? column_groups(c) : cdiv(c->nc, 64);
   if (cells)
     c->compensated ? k_push_cells<R, true><<<cell_blocks, 64 * kSmallWaves, 0, c->stream>>>(p)
@@ -489,6 +492,7 @@ template <class R>
 int stage_push(cpic_context* c, R qdt_2mc, R cdt_dx, R cdt_dy, R cdt_dz, R qsp, int accumulate,
                bool compact, int gather = kGatherRead) {
   StageTimer t(c, CPIC_STAGE_PUSH);
+  c->n_movers = 0;
   if (c->np == 0) return t.finish();
   if (c->D == 0) return fail(CPIC_ERR_INVALID, "particles resident without columns");
   const int blocks = cdiv(c->nc, kBlock);
@@ -676,14 +680,12 @@ int alloc_column_set(cpic_context* c, int D, int M1, int M2, ColumnSet& out) {
     if ((t = alloc((void**)&s.ovf_cell, sizeof(int) * s.ovf_cap))) return t;
     if ((t = alloc((void**)&s.dep, sizeof(unsigned long long) * kDepMasks * words))) return t;
     const size_t groups = c->nc_pad / 64;
-    // (movers: k_push_cells counts per block of kSmallWaves cells)
-    const size_t ints = 3 * groups + (size_t)c->nc_pad / kSmallWaves;
+    const size_t ints = 3 * groups;
     if ((t = alloc((void**)&s.dep_words, sizeof(int) * ints))) return t;
     if (s.MW > (c->nc <= kSmallCells ? kSmallWords : kTakenWords))
       if ((t = alloc((void**)&s.taken, sizeof(unsigned long long) * words))) return t;
     s.rec_flags = s.dep_words + groups;
     s.grp_rows = s.dep_words + 2 * groups;
-    s.grp_movers = s.dep_words + 3 * groups;
     for (int b = 0; b < 2; ++b) {
       if ((t = fill_zero<int>(c, s.cnt[b], c->nc_pad))) return t;
       if ((t = fill_zero<unsigned long long>(c, s.mask[b], words))) return t;
@@ -1144,9 +1146,13 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
                    sizeof(double) * (2 * (size_t)c->partial_rows + 1) * c->n_partials)))
       return bail(s);
     if ((s = alloc((void**)&c->red_out, sizeof(double) * 4))) return bail(s);
-    if ((s = alloc((void**)&c->status, 2 * kStatusStride * sizeof(int)))) return bail(s);
+    // (k_push_cells counts its movers per block of kSmallWaves cells)
+    const size_t n_counts = c->nc_pad / (c->nc <= 2 * kSmallCells ? kSmallWaves : 64);
+    if ((s = alloc((void**)&c->status, (2 * kStatusStride + n_counts) * sizeof(int))))
+      return bail(s);
     c->err = c->status;
     c->ovf_count = reinterpret_cast<unsigned int*>(c->status + kStatusStride);
+    c->cell_movers = c->status + 2 * kStatusStride;
     if (hipHostMalloc((void**)&c->push_host, sizeof(PushStatus), hipHostMallocDefault) !=
         hipSuccess) {
       c->push_host = nullptr;
@@ -1162,7 +1168,8 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
       return CPIC_OK;
     });
     if (s) return bail(s);
-    if (hipMemsetAsync(c->status, 0, 2 * kStatusStride * sizeof(int), c->stream) != hipSuccess ||
+    if (hipMemsetAsync(c->status, 0, (2 * kStatusStride + n_counts) * sizeof(int), c->stream) !=
+            hipSuccess ||
         hipMemsetAsync(c->red_out, 0, sizeof(double) * 4, c->stream) != hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return bail(fail(CPIC_ERR_HIP, "context initialisation failed"));
@@ -1811,13 +1818,10 @@ int cpic_stage_times(cpic_context* c, int64_t* counts, double* ms) {
 int cpic_last_push_movers(cpic_context* c, int64_t* movers) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
-    // counted per block by a tangent push, per group or block by a column push
-    const bool columns = c->D > 0 && c->np > 0;
-    const int* from = columns ? c->grp_movers : c->block_movers;
-    std::vector<int> per((size_t)(columns ? c->n_movers : c->n_block_movers));
+    std::vector<int> per((size_t)c->n_movers);
     if (!per.empty())
-      HIP_TRY(hipMemcpyAsync(per.data(), from, sizeof(int) * per.size(), hipMemcpyDeviceToHost,
-                             c->stream));
+      HIP_TRY(hipMemcpyAsync(per.data(), c->last_movers, sizeof(int) * per.size(),
+                             hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     int64_t sum = 0;
     for (int k : per) sum += k;
