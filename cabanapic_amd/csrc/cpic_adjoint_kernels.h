@@ -353,7 +353,7 @@ __device__ __forceinline__ void streak_bwd(const R pos[3], const R rem[3], R q, 
       llenh += ldsp[k] * (double)dsp0[k];
     }
     // lenh = 0.5 len, len = (dir - mid) / dsp0 on the crossed axis
-    const double lb = 0.5 * llenh * tangent_rcp(crossed);
+    const double lb = tangent_over(0.5 * llenh, crossed);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       double lm = lmid1[k], ld0 = ldsp[k] * (double)lenh;
@@ -387,8 +387,7 @@ __device__ __forceinline__ void displacement_bwd(R ux, R uy, R uz, R cdt_dx, R c
       lu[k] += ld[k] * ((double)v0 * (double)c[k]);
     }
     // v0 = 1 / r, r = sqrt(s), s = 1 + |u|^2: ls 2 u
-    const double ri = tangent_rcp(r);
-    const double ls2 = -lv0 * (double)v0 * ri * ri;
+    const double ls2 = tangent_over(tangent_over(-lv0 * (double)v0, r), r);
 #pragma unroll
     for (int k = 0; k < 3; ++k) lu[k] += ls2 * (double)u[k];
   }
@@ -456,7 +455,7 @@ __device__ __forceinline__ void boris_bwd(const V4& e0, const V4& e1, const V4& 
     // X2 = ux cby - uy cbx
     lu1[0] += lX2 * (double)cby; lcby += lX2 * (double)ux; lu1[1] -= lX2 * (double)cbx; lcbx -= lX2 * (double)uy;
     // v4 = 2 v4a, v4a = v3 / den, den = 1 + v1 v3sq
-    const double lv4a = 2.0 * lv4 * tangent_rcp(den);  // over den
+    const double lv4a = tangent_over(2.0 * lv4, den);  // over den
     lv3 += lv4a;
     const double lden = -lv4a * (double)v4a;
     double lv1 = lden * (double)v3sq;
@@ -474,8 +473,7 @@ __device__ __forceinline__ void boris_bwd(const V4& e0, const V4& e1, const V4& 
     lcby += lv1 * 2.0 * (double)cby;
     lcbz += lv1 * 2.0 * (double)cbz;
     // v0 = qdt_2mc / r, r = sqrt(s), s = 1 + |u1|^2
-    const double ri = tangent_rcp(r);
-    const double ls2 = -lv0 * (double)v0 * ri * ri;
+    const double ls2 = tangent_over(tangent_over(-lv0 * (double)v0, r), r);
     lu1[0] += ls2 * (double)ux;
     lu1[1] += ls2 * (double)uy;
     lu1[2] += ls2 * (double)uz;
