@@ -40,16 +40,19 @@ class HostRing {
     static HostRing ring;
     return ring;
   }
+  // A context is opened (closed).  Neither waits for a download, which holds the
+  // ring as long as the work queued before it runs: the last context to be closed
+  // finds the ring free.
   void retain() {
-    std::lock_guard<std::mutex> l(m_);
+    std::lock_guard<std::mutex> l(users_mutex_);
     ++users_;
   }
   void release() {
-    std::lock_guard<std::mutex> l(m_);
-    if (--users_ == 0 && ring_) {
-      (void)hipHostFree(ring_);
-      ring_ = nullptr;
-    }
+    std::lock_guard<std::mutex> l(users_mutex_);
+    if (--users_ > 0) return;
+    std::lock_guard<std::mutex> r(m_);
+    if (ring_) (void)hipHostFree(ring_);
+    ring_ = nullptr;
   }
 
   // n bytes of device memory into dst, after the work queued on the stream;
@@ -61,8 +64,9 @@ class HostRing {
   }
 
  private:
-  std::mutex m_;
+  std::mutex users_mutex_;  // taken before m_ where both are
   int users_ = 0;
+  std::mutex m_;  // held while the ring is in use
   char* ring_ = nullptr;
 
   static hipError_t plain(void* dst, const void* src, size_t n, hipStream_t stream) {
