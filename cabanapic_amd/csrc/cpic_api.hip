@@ -605,7 +605,7 @@ template <class R>
 int launch_field_energy(cpic_context* c, double* out) {
   const bool es = c->solver == CPIC_FIELD_SOLVER_ES_1D;
   const long n = es ? c->ncells : c->nx * c->ny * c->nz;
-  const int blocks = std::max(1, std::min(cdiv(n, kBlock), c->n_partials));
+  const int blocks = reduce_blocks(n);
   if (es)
     k_es_energy_partial<R><<<blocks, kBlock, 0, c->stream>>>((const R*)c->fields, c->grid,
                                                              c->partials);
@@ -621,7 +621,7 @@ int launch_kinetic(cpic_context* c, double scale, double* out) {
   double* part = c->partials + 2 * (size_t)c->partial_rows * c->n_partials;
   int blocks = 1;
   if (c->D > 0 && c->np > 0) {
-    blocks = std::max(1, std::min(cdiv(c->nc, kBlock), c->n_partials));
+    blocks = reduce_blocks(c->nc);
     const ColState<R> cs = col_state<R>(c, c->cur);
     k_kinetic_columns<R><<<blocks, kBlock, 0, c->stream>>>(cs, (int)c->nc, part);
   } else {
@@ -1126,8 +1126,8 @@ int cpic_create(const cpic_config* cfg, cpic_context** out) {
     c->cg.nc = (int)c->nc;
     c->cg.sy = (int)X;
     c->cg.sz = (int)(X * Y);
-    // one block's partial per kBlock cells (voxels for the ES energy), and as
-    // many steps' sets as 4 MB hold, 64 at most
+    // one block's partial per kBlock cells (k_advance_b_energy; voxels for the ES
+    // energy), and as many steps' sets as 4 MB hold, 64 at most
     c->n_partials = cdiv(c->ncells, kBlock);
     c->partial_rows = std::clamp((int)((4L << 20) / (16L * c->n_partials)), 1, 64);
   

@@ -7,7 +7,6 @@
 // device and kept.  Calls that overlap on one GPU share the array and race.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <mutex>
 
 #include "../../include/cabanapic_amd.h"
@@ -22,10 +21,9 @@ using cpic_detail::fail_msg;
 
 namespace {
 
-// At most this many blocks write partials: the grid-stride kernel covers any
-// grid with them, so the array does not grow with the grid.
-constexpr int kScratchBlocks = 4096;
-constexpr int kScratchDoubles = 2 * kScratchBlocks;  // [block][E, B]: 64 KiB
+// The blocks' number is bounded (reduce_blocks), so the array does not grow with
+// the grid.
+constexpr int kScratchDoubles = 2 * kReduceBlocks;  // [block][E, B]: 64 KiB
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
@@ -58,7 +56,7 @@ hipError_t scratch_on_current_device(double** out) {
 template <class R>
 hipError_t launch(const void* fields, const Grid& g, double* part, double* out, hipStream_t st) {
   const long n = (long)g.nx * g.ny * g.nz;
-  const int blocks = (int)std::max(1L, std::min((n + kBlock - 1) / kBlock, (long)kScratchBlocks));
+  const int blocks = reduce_blocks(n);
   k_field_energy_partial<R><<<blocks, kBlock, 0, st>>>((const R*)fields, g, part);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -74,7 +72,7 @@ extern "C" int cpic_field_energies_noalloc(const void* fields, int32_t real_size
   if (real_size != 4 && real_size != 8) return fail_msg(CPIC_ERR_INVALID, "real_size must be 4 or 8");
   if (nx < 1 || ny < 1 || nz < 1) return fail_msg(CPIC_ERR_INVALID, "grid extents must be >= 1");
   // the voxel indexing of the kernels is 32-bit, as for a context; the
-  // partials do not grow with the grid (at most kScratchBlocks blocks)
+  // partials do not grow with the grid (at most kReduceBlocks blocks)
   const double ng = (double)(nx + 2) * (double)(ny + 2) * (double)(nz + 2);
   if (ng * 9 > 2147483647.0)
     return fail_msg(CPIC_ERR_INVALID, "grid too large for 32-bit voxel indexing");
