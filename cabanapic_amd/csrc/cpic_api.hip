@@ -1350,14 +1350,16 @@ int download_particles(cpic_context* c, int64_t n, void* x, void* y, void* z, vo
   const size_t rs = c->rsz();
   const size_t nc = (size_t)c->nc;
   Scratch stage;
-  const size_t bytes = sizeof(long long) * nc + (7 * rs + sizeof(int) + sizeof(long long)) * n;
-  if (int s = alloc(&stage.p, bytes)) return s;
+  // (the cells' counts share the particles' part, which few particles in many
+  // cells would not fill)
+  const size_t part = std::max((7 * rs + sizeof(int) + sizeof(long long)) * n, sizeof(int) * nc);
+  if (int s = alloc(&stage.p, sizeof(long long) * nc + part)) return s;
   char* sp = (char*)stage.p;
   long long* first_dev = (long long*)sp;
   char* soa = sp + sizeof(long long) * nc;
   int* cell_dev = (int*)(soa + 7 * rs * n);
   long long* tag_dev = (long long*)(cell_dev + n);
-  int* occ_dev = (int*)soa;  // the counts use the SoA area before the gather
+  int* occ_dev = (int*)soa;  // before the gather
   std::vector<int> occ(nc);
   k_column_occupancy<<<cdiv(c->nc, kBlock), kBlock, 0, c->stream>>>(
       c->cnt[c->cur], c->mask[c->cur], (int)c->nc, (int)c->nc_pad, c->D, occ_dev);
