@@ -349,13 +349,23 @@ bool small_grid(const cpic_context* c) {
 }
 
 // Whether this push packs the columns: every interval-th one that the caller
-// names, by default every kCompactInterval-th of a grid that fills the chip.
-// Packing walks a column with one wave, and arrivals keep filling the lowest
-// holes, so that the columns of a small grid stay short without it.
+// names, else every kCompactInterval-th: on a grid that fills the chip whatever
+// the columns hold, and on a smaller one if they hold mostly holes, that is if
+// the longest of them is, but for one mask word, twice as long as the mean.
+// Packing walks a column with one wave.  Where arrivals keep filling the lowest
+// holes the columns of a small grid stay short without it: over 1600 steps no
+// plasma was slower (32 cells x 64 in FP64 30 us a step instead of 33, 200 x 100
+// 37 and 42, 32^3 x 32 two-stream 66 to 97 and 68 to 99, 48^3 x 32 153 to 198 and
+// 153 to 201).  But the rows of a crowd stay in use until their last particle
+// leaves: 8000 particles that started in one cell of 20^3 took 164 us a push, and
+// take 38 after the 33rd, which packs them.
+// (After check_headroom, which leaves the last push's rows in push_host.)
 bool packs_now(cpic_context* c, int interval) {
   const long n = c->pushes++;
-  if (interval <= 0 && cdiv(c->nc, 64) < 2048) return false;
-  return n % (interval > 0 ? interval : kCompactInterval) == 0;
+  if (interval > 0) return n % interval == 0;
+  if (n % kCompactInterval) return false;
+  if (cdiv(c->nc, 64) >= 2048) return true;
+  return n > 0 && c->push_host->rows > 2 * (c->np / c->nc) + 64;
 }
 
 template <class R, bool K>

@@ -75,8 +75,9 @@ typedef struct cpic_step_params {
                                the reference dumps every step
                                (ENERGY_DUMP_INTERVAL, example.cpp:53-55)   */
   int32_t compact_interval; /* particles stay binned by cell; every k-th
-                               push also packs each cell's column
-                               (0 = every 32nd push)                         */
+                               push also packs each cell's column (0 = every
+                               32nd; on grids of up to 131008 cells only if
+                               the columns hold mostly holes)                */
   int32_t kinetic_interval; /* kinetic energy every k steps (0 = never)     */
 } cpic_step_params;
 
@@ -143,8 +144,8 @@ int cpic_clear_accumulator_array(cpic_context *ctx);
 /* push<ScatterView> with the inline move_p, src/push.h:7-300,
  * src/move_p.h:59-374: Boris push, cell crossing and charge-conserving
  * deposit, added to the accumulators as the reference's push does.  The
- * first push after an upload and every 32nd one also pack the particle
- * columns (no visible effect but the order within a cell).  boundary must be
+ * pushes that compact_interval = 0 names also pack the particle columns (no
+ * visible effect but the order within a cell).  boundary must be
  * CPIC_BOUNDARY_PERIODIC. */
 int cpic_push(cpic_context *ctx, double qdt_2mc, double cdt_dx,
               double cdt_dy, double cdt_dz, double qsp, int32_t boundary);
