@@ -1402,6 +1402,7 @@ int download_particles(cpic_context* c, int64_t n, void* x, void* y, void* z, vo
     if (dst[k]) HIP_TRY(ring.copy(dst[k], soa + k * rs * n, rs * n, c->stream));
   if (cell) HIP_TRY(ring.copy(cell, cell_dev, sizeof(int) * n, c->stream));
   if (tag) HIP_TRY(ring.copy(tag, tag_dev, sizeof(long long) * n, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
   return CPIC_OK;
 }
 
@@ -1471,7 +1472,10 @@ int cpic_download_fields(cpic_context* c, void* f) {
   return guarded([&]() -> int {
     if (int s = check_ctx(c)) return s;
     if (!f) return fail(CPIC_ERR_INVALID, "null fields");
-    HIP_TRY(HostRing::get().copy(f, c->fields, c->rsz() * 9 * c->ncells, c->stream));
+    const size_t n = c->rsz() * 9 * c->ncells;
+    if (n > HostRing::kTiny) HIP_TRY(HostRing::get().copy(f, c->fields, n, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (n <= HostRing::kTiny) HIP_TRY(hipMemcpy(f, c->fields, n, hipMemcpyDeviceToHost));
     return CPIC_OK;
   });
 }

@@ -1,7 +1,7 @@
 """The pinned download ring against a stand-in for the runtime, on the CPU: a
 download that waits for the work queued before it keeps no other thread from
-opening or closing a context, the data arrive whole, and the ring is given back
-with the last context."""
+opening or closing a context, one too small for the ring is left queued, the data
+arrive whole, and the ring is given back with the last context."""
 import os
 import subprocess
 
@@ -70,10 +70,13 @@ PROGRAM = r"""
 #include <future>
 int main(int, char** argv) {
   const size_t n = atol(argv[1]);
-  std::vector<char> src(n), dst(n);
+  std::vector<char> src(n), dst(n), small(4096);
   for (size_t i = 0; i < n; ++i) src[i] = (char)(i * 31 + i / 4096);
   cpic::HostRing& ring = cpic::HostRing::get();
   ring.retain();
+  auto queued = std::async(std::launch::async,
+                           [&] { return ring.copy(small.data(), src.data(), small.size(), nullptr); });
+  const bool at_once = queued.wait_for(std::chrono::seconds(10)) == std::future_status::ready;
   auto download = std::async(std::launch::async, [&] { return ring.copy(dst.data(), src.data(), n, nullptr); });
   {
     std::unique_lock<std::mutex> l(gate.m);
@@ -86,11 +89,12 @@ int main(int, char** argv) {
     gate.open = true;
     gate.cv.notify_all();
   }
-  const bool ok = download.get() == hipSuccess;
+  const bool ok = download.get() == hipSuccess && queued.get() == hipSuccess &&
+                  memcmp(small.data(), src.data(), small.size()) == 0;
   other.get();
   const int held = gate.allocated;
   ring.release();
-  printf("%d %d %d %d %d\n", free, ok, src == dst, held, gate.allocated);
+  printf("%d %d %d %d %d %d\n", at_once, free, ok, src == dst, held, gate.allocated);
 }
 """
 
@@ -106,4 +110,4 @@ def test_contexts_come_and_go_during_a_download(tmp_path, size):
                     "-o", exe, str(tmp_path / "main.cpp")], check=True)
     out = subprocess.run([exe, str(size)], check=True, capture_output=True, text=True, timeout=60)
     # nothing waited, success, the right bytes, one ring held and then none
-    assert out.stdout.split() == ["1", "1", "1", "1", "0"]
+    assert out.stdout.split() == ["1", "1", "1", "1", "1", "0"]
