@@ -26,6 +26,21 @@
 
 using namespace cpic;
 
+// The ring's pieces.  Slots begin on whole pieces; the source is aligned as the
+// array that it is a part of.
+hipError_t cpic::launch_to_pinned(void* pinned, const void* src, size_t n, hipStream_t stream) {
+  const int blocks = (int)std::min<size_t>(n / (16 * kCopyAtOnce * kBlock) + 1, 128);
+  char* const d = (char*)pinned;
+  const char* const s = (const char*)src;
+  if ((uintptr_t)src % 16 == 0)
+    k_to_pinned<uint4><<<blocks, kBlock, 0, stream>>>(d, s, n);
+  else if ((uintptr_t)src % 4 == 0)
+    k_to_pinned<unsigned><<<blocks, kBlock, 0, stream>>>(d, s, n);
+  else
+    k_to_pinned<unsigned char><<<blocks, kBlock, 0, stream>>>(d, s, n);
+  return hipGetLastError();
+}
+
 namespace {
 
 thread_local std::string g_last_error;

@@ -3,9 +3,15 @@
 // The runtime's own pageable copy runs at 10.5 GB/s into memory that has just
 // been allocated (one thread moves the data out of a staging buffer and takes
 // the page faults): 7.9 ms for the 79 MB of fields of a 128^3 grid, an eighth
-// of 24 steps.  Here the copy engine fills 2 MB pieces of a pinned ring while
-// up to four threads empty it: 2.2 ms (36 GB/s; 50 MB 5.0 -> 1.5 ms).  1 MB
-// pieces reach 29 GB/s, one thread 14, six threads no more.
+// of 24 steps.  Here 2 MB pieces of a pinned ring are filled while up to four
+// threads empty it: 2.2 ms (36 GB/s; 50 MB 5.0 -> 1.5 ms), 1.7 into memory that is
+// there (47 GB/s).  1 MB pieces reach 29 GB/s, one thread 14, six threads no more.
+//
+// A kernel fills them, not a copy engine: the driver clears device memory that is
+// given back with the copy engines, 30 ms for each GB, and what they copy
+// meanwhile moves at 12 GB/s instead of 45 (79 MB 6.6 ms, by the kernel 1.7; a
+// gradient of 64^3 x 32, 4 steps, by an Adjoint made for it 64 ms, by the kernel
+// 38).
 //
 // The caller is one of the threads, and the only one below 16 MB, where others
 // gain little (7 MB 0.45 against 0.5 ms) and cost much where the program's own
@@ -25,6 +31,9 @@
 #include <vector>
 
 namespace cpic {
+
+// n bytes of device memory into pinned memory, by a kernel on the stream.
+hipError_t launch_to_pinned(void* pinned, const void* src, size_t n, hipStream_t stream);
 
 // The pinned ring, one for the process: allocated by the first large download
 // and given back with the last context.  A second thread's download at the
@@ -96,8 +105,8 @@ class HostRing {
   static int threads_for(size_t n) { return n < (16u << 20) ? 1 : n < (32u << 20) ? 2 : kThreads; }
 
   // Piece i goes through slot i % kPieces and is thread i % threads's, which
-  // empties the slot and then has the copy engine fill it with the next piece of
-  // the slot, its own too: the threads share nothing but the stream.
+  // empties the slot and then has it filled with the next piece of the slot, its
+  // own too: the threads share nothing but the stream.
   hipError_t ringed(char* dst, const char* src, size_t n, hipStream_t stream) {
     const long pieces = (long)((n + kPiece - 1) / kPiece);
     const int threads = threads_for(n);
@@ -110,8 +119,7 @@ class HostRing {
     auto size = [&](long i) { return std::min(kPiece, n - (size_t)i * kPiece); };
     auto slot = [&](long i) { return ring_ + (size_t)(i % kPieces) * kPiece; };
     auto fill = [&](long i) {
-      hipError_t e = hipMemcpyAsync(slot(i), src + (size_t)i * kPiece, size(i),
-                                    hipMemcpyDeviceToHost, stream);
+      hipError_t e = launch_to_pinned(slot(i), src + (size_t)i * kPiece, size(i), stream);
       if (e == hipSuccess) e = hipEventRecord(ev[i % kPieces], stream);
       if (e != hipSuccess) failure = (int)e;
     };

@@ -41,6 +41,30 @@ template <class R> struct Vec4T;
 template <> struct Vec4T<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct Vec4T<double> { typedef double type __attribute__((ext_vector_type(4))); };
 
+// n bytes to pinned host memory, as many Ts as they hold and then the rest; both
+// pointers aligned to T.  A thread has kCopyAtOnce loads in flight.
+constexpr int kCopyAtOnce = 4;
+template <class T>
+__global__ void __launch_bounds__(kBlock) k_to_pinned(char* __restrict__ dst, const char* __restrict__ src, size_t n) {
+  const size_t count = n / sizeof(T), stride = (size_t)gridDim.x * blockDim.x;
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  T* const out = reinterpret_cast<T*>(dst);
+  const T* const in = reinterpret_cast<const T*>(src);
+  for (size_t i0 = t; i0 < count; i0 += kCopyAtOnce * stride) {
+    T v[kCopyAtOnce];
+#pragma unroll
+    for (int u = 0; u < kCopyAtOnce; ++u) {
+      const size_t i = i0 + u * stride;
+      v[u] = in[i < count ? i : count - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < kCopyAtOnce; ++u)
+      if (i0 + u * stride < count) out[i0 + u * stride] = v[u];
+  }
+  const size_t rest = count * sizeof(T) + t;
+  if (rest < n) dst[rest] = src[rest];
+}
+
 struct Grid {
   int nx, ny, nz;
   int sy, sz;  // voxel strides along y and z (x stride is 1)

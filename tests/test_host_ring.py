@@ -68,6 +68,9 @@ PROGRAM = r"""
 #include <chrono>
 #include <cstdio>
 #include <future>
+hipError_t cpic::launch_to_pinned(void* d, const void* s, size_t n, hipStream_t st) {
+  return hipMemcpyAsync(d, s, n, hipMemcpyDeviceToHost, st);
+}
 int main(int, char** argv) {
   const size_t n = atol(argv[1]);
   std::vector<char> src(n), dst(n), small(4096);
