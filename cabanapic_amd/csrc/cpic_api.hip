@@ -334,7 +334,10 @@ int column_groups(const cpic_context* c) { return (int)(c->nc_pad / 64); }
 // 2 in us, with 2, 4 and 8 waves: 32^3 cells x 32 (512 groups) 45 29 25 / 23
 // 18 16; 48^3 x 32 (1728) 87 85 85 / 44 46 58; 128^3 x 32 (32768) 1324 1281
 // 1347 / 724 726 998; 1D, 32 cells x 64 in FP64, 95 58 42 / 41 31 26.  (One
-// wave: 1359 / 731 at 128^3.)
+// wave: 1359 / 731 at 128^3.)  Just above the line both splits take the same
+// time, then 4 and 2 waves less; with those and with 8 and 8: 34x32x32 x 32 (544
+// groups) 33 24 and 33 24, 36^3 x 32 (729) 35 26 and 36 26, in FP64 68 30 and 74
+// 39, 40^3 x 32 (1000) 45 28 and 46 31, 44^3 x 32 (1331) 67 36 and 66 44.
 struct SplitWaves {
   int push, arrive;
 };

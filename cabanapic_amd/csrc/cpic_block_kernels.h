@@ -6,14 +6,15 @@
 // at most a thread per cell.  On a 1D deck they took 21 of a step's 50 us: each
 // launch starts with cold caches and drains before the next.  Up to
 // kBlockThreads cells one workgroup runs them all, with barriers in the
-// launches' places: 11 us for 32 cells, and a step, with the push's status sent
-// to the host before the field stages, 50 -> 40 us in FP64.  Every value is
-// computed by the same operations, and every sum in the same order, as in the
-// kernels that larger grids run.
+// launches' places: 11 us for 32 cells, of the 30 us that a step of 32 cells x 64
+// takes in FP64 now (the host, to which the push's status goes before the field
+// stages, queues the next step meanwhile).  Every value is computed by the same
+// operations, and every sum in the same order, as in the kernels that larger grids
+// run.
 //
 // (The particle passes stay outside: with whole steps in one workgroup the same
-// deck took 60 us a step, bound by its CU's vector cache, to which the rows of
-// a cell, a wave's lanes, are 64 lines.)
+// deck took 60 us a step, where separate launches took 50, bound by its CU's
+// vector cache, to which the rows of a cell, a wave's lanes, are 64 lines.)
 //
 // Visibility: what passes from wave to wave here goes through one CU's
 // write-through vector cache, where a barrier is enough.  What atomics change

@@ -7,8 +7,8 @@
 // threads empty it: 2.2 ms (36 GB/s; 50 MB 5.0 -> 1.5 ms), 1.7 into memory that is
 // there (47 GB/s).  1 MB pieces reach 29 GB/s, one thread 14, six threads no more.
 //
-// A kernel fills them, not a copy engine: the driver clears device memory that is
-// given back with the copy engines, 30 ms for each GB, and what they copy
+// A kernel fills them, not a copy engine: the GPU driver clears device memory that
+// is given back with the copy engines, 30 ms for each GB, and what they copy
 // meanwhile moves at 12 GB/s instead of 45 (79 MB 6.6 ms, by the kernel 1.7; a
 // gradient of 64^3 x 32, 4 steps, by an Adjoint made for it 64 ms, by the kernel
 // 38).

@@ -1,8 +1,7 @@
-"""Steps that run in one workgroup, and steps whose stages after the particle
-passes do, against the launches of the general path (which a timed stage
-selects): everything that a run leaves equals bit for bit.  Sizes at the limits
-of both (256 and 1024 cells, and one more), partly filled waves and blocks,
-one cell, several calls, steps past one launch's limit, particles fast enough
+"""Steps whose stages after the particle passes run in one workgroup, against the
+launches of the general path (which a timed stage selects): everything that a run
+leaves equals bit for bit.  Sizes at the limit of 1024 cells and one more, partly
+filled waves and blocks, one cell, several calls, many steps, particles fast enough
 for records of every crossing and for the overflow list."""
 import numpy as np
 import pytest

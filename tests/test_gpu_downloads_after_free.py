@@ -1,5 +1,5 @@
-"""A large download does not wait for the driver to clear memory that was given
-back before it (the driver uses the copy engines for that): right after a context
+"""A large download does not wait for the GPU driver to clear memory given
+back before it (it uses the copy engines for that): right after a context
 of some GB is closed it takes the time that it takes at rest."""
 import ctypes
 import time
