@@ -500,7 +500,8 @@ template <class R> struct RowCursor {
     }
   }
   __device__ int next(const ColState<R>& cs, int ci) {
-    for (int guard = 0; guard < 64; ++guard) {
+    // (every turn returns, goes to the next word or ends the search for holes)
+    for (int guard = 0; guard < cs.MW + 2; ++guard) {
       if (!append) {
         if (have && freeb) {
           const int b = __ffsll((long long)freeb) - 1;
