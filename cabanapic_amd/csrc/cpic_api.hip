@@ -1038,9 +1038,10 @@ int launch_tail_step(cpic_context* c, const cpic_step_params* sp, int gather, bo
 // nsteps iterations of the loop body of example/example.cpp:216-279 on the
 // context's stream, no host synchronisation; energies of step s (1-based)
 // into dhist row s - 1 (3 doubles: E, B, kinetic) when dhist is not null,
-// as sp's energy and kinetic intervals ask.
+// as sp's energy and kinetic intervals ask of step before + s of the run.
 template <class R>
-int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, double* dhist) {
+int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, double* dhist,
+              int64_t before = 0) {
   const int ei = sp->energy_interval;
   const int ki = sp->kinetic_interval;
   const R px = (R)sp->px, py = (R)sp->py, pz = (R)sp->pz;
@@ -1065,7 +1066,8 @@ int run_steps(cpic_context* c, const cpic_step_params* sp, int64_t nsteps, doubl
     // needed while ghost accumulators may hold data
     if (!c->acc_ghosts_zero && (t = stage_clear<R>(c))) return t;
     if ((t = check_headroom(c))) return t;
-    const bool do_e = ei > 0 && step % ei == 0, do_k = ki > 0 && step % ki == 0;
+    const bool do_e = ei > 0 && (before + step) % ei == 0;
+    const bool do_k = ki > 0 && (before + step) % ki == 0;
     double* row = dhist ? dhist + 3 * (step - 1) : c->red_out;
     const bool compact = packs_now(c, sp->compact_interval);
     const int gather = !fused ? kGatherRead : step == nsteps ? kGatherStore : kGatherFields;
