@@ -44,11 +44,9 @@ def test_tangent(dtype):
 def test_adjoint(dtype):
     st, _, fast = _state(dtype)
     seed = np.random.default_rng(23).standard_normal((6, st.np))
-    with sim_from_state(st) as sim:
-        adj = Adjoint(sim)
+    with sim_from_state(st) as sim, Adjoint(sim) as adj:
         adj.forward(states.step_consts(dtype), 1, 1)
         gf, gp = adj.backward(np.zeros((9, st.ng)), seed)
-        adj.close()
         assert sim.device_errors() == 0
     assert np.isfinite(gp).all() and np.isfinite(gf).all()
     assert_same_bits(gp[:, fast] + 0.0, seed[:, fast], "adjoints")
